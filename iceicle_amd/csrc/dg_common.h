@@ -513,11 +513,12 @@ __device__ __forceinline__ void interior_point_flux_split(const typename PH::Par
     using R = typename PH::real;
     R fadv[M], fvis[M], gddg[M * D], uavg[M];
     PH::conv(ph, uL, uR, nrm, fadv);
+    const R penalty = ph.beta0 * recip(h);
 #pragma unroll
     for (int v = 0; v < M; ++v) {
-        const R jump = jmp ? jmp[v] : uR[v] - uL[v];
+        const R jump = (jmp ? jmp[v] : uR[v] - uL[v]) * penalty;
 #pragma unroll
-        for (int d = 0; d < D; ++d) gddg[v * D + d] = ph.beta0 * jump / h * nrm[d] + gs[v * D + d];
+        for (int d = 0; d < D; ++d) gddg[v * D + d] = jump * nrm[d] + gs[v * D + d];
         uavg[v] = R(0.5) * (uL[v] + uR[v]);
     }
     PH::diff(ph, uavg, gddg, nrm, fvis);

@@ -15,7 +15,8 @@
 #include "engine.h"
 #include "kernels.h"
 #include "mesh.hpp"
-#include "physics_dev.h"
+#include "physics_params.h"
+#include "stage.h"
 #include "fields.h"
 
 namespace {
@@ -507,6 +508,15 @@ static int space_create(const ice_mesh_desc* mds, int nmesh, const ice_space_des
         }
         s->efaces.assign((size_t)m.nelem * 2 * D, -1);
         const int nfi = (int)s->fint.size(), nfb = (int)s->fbdy.size();
+        // structured elements meet across opposite faces with the tangential
+        // axes aligned, which the one-launch kernels assume
+        for (const int4& r : s->fint) {
+            const int fnl = r.z & 7, fnr = (r.z >> 3) & 7, orient = (r.z >> 6) & 7;
+            const signed char* tl = &s->ftens[((size_t)fnl * no + 0) * s->nfq];
+            const signed char* tr = &s->ftens[((size_t)fnr * no + orient) * s->nfq];
+            if (fnr != (fnl + D) % (2 * D) || std::memcmp(tl, tr, s->nfq) != 0)
+                throw ice::Error{ICE_ERR_UNSUPPORTED, "elements of a structured mesh are not aligned"};
+        }
         for (int f = 0; f < nfi; ++f) {
             const int4 r = s->fint[f];
             const int fnl = r.z & 7, fnr = (r.z >> 3) & 7, orient = (r.z >> 6) & 7;
@@ -1190,6 +1200,9 @@ struct ice_stepper {
 
 namespace {
 
+// textbook RK3-SSP increments in each stage's combination
+constexpr double C1[1] = {1.0}, C2[2] = {0.25, 0.25}, C3[3] = {1.0 / 6.0, 1.0 / 6.0, 2.0 / 3.0};
+
 int step_once(ice_stepper* S, double* u, hipStream_t st) {
     ice_disc* d = S->disc;
     const ice_space* sp = d->space;
@@ -1220,6 +1233,17 @@ int step_once(ice_stepper* S, double* u, hipStream_t st) {
             axpy(1.0 / 6.0, k1, u);
             axpy(1.0 / 6.0, k1, u);
             axpy(2.0 / 3.0, k1, u);
+        } else if (ice::wave2d_covers(sp->ndim, sp->p, d->dd)) {
+            // a launch per stage: residual, increment and combination; no
+            // stage may write the state it reads, so the third's is in k3
+            auto stage = [&](const double* x, double* k, int nprev, const double* c, double* out, bool store_k) {
+                const double* kk[2] = {k1, k2};
+                const auto cb = ice::make_stage<double>(u, nprev, kk, c, dt, S->dte, S->st, out, store_k);
+                rc |= ice::residual_stage(sp->ndim, sp->p, d->prm.flux, sp->dev, d->ph, d->dd, x, k, cb, st);
+            };
+            stage(u, k1, 0, C1, us, true);
+            stage(us, k2, 1, C2, k3, true);
+            stage(k3, res, 2, C3, u, false);
         } else {
             // ssp_rk3.hpp:164-190; each stage's increment and combination
             // u1 = u + dt k1, u2 = u + dt (k1 + k2)/4, u = u + dt (k1/6 + k2/6 + 2 k3/3)
@@ -1230,13 +1254,12 @@ int step_once(ice_stepper* S, double* u, hipStream_t st) {
                                                S->st, out, store_k, st);
             };
             const double* k12[2] = {k1, k2};
-            const double c1[1] = {1.0}, c2[2] = {0.25, 0.25}, c3[3] = {1.0 / 6.0, 1.0 / 6.0, 2.0 / 3.0};
             R(u);
-            minv_combine(k1, 0, k12, c1, us, true);
+            minv_combine(k1, 0, k12, C1, us, true);
             R(us);
-            minv_combine(k2, 1, k12, c2, us, true);
+            minv_combine(k2, 1, k12, C2, us, true);
             R(us);
-            minv_combine(k3, 2, k12, c3, u, false);
+            minv_combine(k3, 2, k12, C3, u, false);
         }
         break;
     case ICE_STEP_RK3_TVD: {
@@ -1282,17 +1305,25 @@ int step_once(ice_stepper* S, float* u, hipStream_t st) {
                                            S->st, out, store_k, st);
     };
     const float* kk[2] = {k1, k2};
-    const double c1[1] = {1.0}, c2[2] = {0.25, 0.25}, c3[3] = {1.0 / 6.0, 1.0 / 6.0, 2.0 / 3.0};
     rc |= ice::launch_step_begin(S->st, d->d_wave, S->ctl, st);
-    R(u);
-    if (S->desc.kind == ICE_STEP_RK3_SSP) {
-        minv_combine(k1, 0, kk, c1, us, true);
+    if (S->desc.kind == ICE_STEP_RK3_SSP && ice::wave2d_covers(sp->ndim, sp->p, d->dd)) {
+        auto stage = [&](const float* x, float* k, int nprev, const double* c, float* out, bool store_k) {
+            const auto cb = ice::make_stage<float>(u, nprev, kk, c, dt, S->dte, S->st, out, store_k);
+            rc |= ice::residual_stage(sp->ndim, sp->p, d->prm.flux, sp->dev, d->ph, d->dd, x, k, cb, st);
+        };
+        stage(u, k1, 0, C1, us, true);
+        stage(us, k2, 1, C2, k3, true);
+        stage(k3, us, 2, C3, u, false);
+    } else if (S->desc.kind == ICE_STEP_RK3_SSP) {
+        R(u);
+        minv_combine(k1, 0, kk, C1, us, true);
         R(us);
-        minv_combine(k2, 1, kk, c2, us, true);
+        minv_combine(k2, 1, kk, C2, us, true);
         R(us);
-        minv_combine(k3, 2, kk, c3, u, false);
+        minv_combine(k3, 2, kk, C3, u, false);
     } else {
-        minv_combine(k1, 0, kk, c1, u, false);
+        R(u);
+        minv_combine(k1, 0, kk, C1, u, false);
     }
     rc |= ice::launch_step_end(S->st, st);
     return rc;

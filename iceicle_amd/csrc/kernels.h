@@ -87,6 +87,9 @@ struct StepControl {
     long long ntime;
 };
 
+template <class KT>
+struct StageComb;  // stage.h
+
 // Projection right-hand side b = sum_q f(x_q) phi_i w detJ (projection.hpp:83-110)
 int projection_rhs(int ndim, int p, int neq, const DevSpace& S, const ice_field* f, double* b, hipStream_t st);
 // Per-element squared L2 error terms (l2_error.hpp:37-94)
@@ -116,6 +119,15 @@ int launch_axpby(size_t n, double a, const double* x, double b, double* y, hipSt
 int launch_widen(size_t n, const float* x, double* y, hipStream_t st);  // y = (double)x
 int launch_step_begin(StepState* s, unsigned long long* wave, const StepControl& c, hipStream_t st);
 int launch_step_end(StepState* s, hipStream_t st);
+
+// One-launch 2D residual (residual_wave2d.h); with cb.out the stage form:
+// K = M^-1 R(U) and the stage combination, U not aliasing cb.out.
+inline bool wave2d_covers(int ndim, int p, const DiscDev& dd) { return ndim == 2 && p <= 3 && !dd.Pic; }
+int residual_stage(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
+                   const double* U, double* K, const StageComb<double>& cb, hipStream_t st);
+int residual_stage(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
+                   const float* U, float* K, const StageComb<float>& cb, hipStream_t st);
+int launch_wave_reduce(const double* part, int n, unsigned long long* wave, hipStream_t st);
 
 int residual_fp64(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                   const double* U, double* R, hipStream_t st, hipEvent_t* ev = nullptr);

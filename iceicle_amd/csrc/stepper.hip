@@ -14,6 +14,7 @@
 
 #include "kernels.h"
 #include "physics_dev.h"
+#include "stage.h"
 
 namespace ice {
 
@@ -49,60 +50,6 @@ __device__ __forceinline__ double q1_det(const double* __restrict__ Xe, const do
     else
         return J[0][0] * (J[1][1] * J[2][2] - J[1][2] * J[2][1]) - J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) +
                J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0]);
-}
-
-// Optional stage combination formed by the kernel from the increment k_new
-// it computes: out = base + dt (c0 k0 + c1 k1 + cn k_new) over the nprev
-// earlier increments k0, k1, with the step of rk_combine_kernel (the
-// stepper's dt, or the element's, none once the run is done); k_new is
-// rounded to KT first, as when it is stored and read back.
-template <class KT>
-struct StageComb {
-    KT* out = nullptr;  // null: k = M^-1 r only
-    const KT* base = nullptr;
-    const KT* k0 = nullptr;
-    const KT* k1 = nullptr;
-    int nprev = 0;
-    double c0 = 0, c1 = 0, cn = 0;
-    const double* dtp = nullptr;
-    const double* dte = nullptr;
-    const StepState* stp = nullptr;
-    bool store_k = true;  // also store k_new (a later stage reads it)
-};
-
-// out = base + dt (c0 k0 + c1 k1 + cn kn) over the NL contiguous values of a
-// line at o, with NPV earlier increments: straight-line loads of each input
-// (so they merge into wide loads), all read before out, which may be base,
-// is stored; then kn itself if the stage keeps it
-template <int NPV, int NL, class KT>
-__device__ __forceinline__ void stage_combine_line(const StageComb<KT>& cb, KT* __restrict__ k, size_t o, double dt,
-                                                   const KT* kn) {
-    double sum[NL], bv[NL];
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-        double acc = 0.0;
-        if constexpr (NPV > 0) acc = cb.c0 * (double)cb.k0[o + i];
-        if constexpr (NPV > 1) acc += cb.c1 * (double)cb.k1[o + i];
-        sum[i] = acc;
-        bv[i] = (double)cb.base[o + i];
-    }
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-        sum[i] += cb.cn * (double)kn[i];
-        cb.out[o + i] = (KT)(bv[i] + dt * sum[i]);
-    }
-    if (cb.store_k) {
-#pragma unroll
-        for (int i = 0; i < NL; ++i) k[o + i] = kn[i];
-    }
-}
-
-template <int NL, class KT>
-__device__ __forceinline__ void stage_combine_line(const StageComb<KT>& cb, KT* __restrict__ k, size_t o, double dt,
-                                                   const KT* kn) {
-    if (cb.nprev == 0) stage_combine_line<0, NL, KT>(cb, k, o, dt, kn);
-    else if (cb.nprev == 1) stage_combine_line<1, NL, KT>(cb, k, o, dt, kn);
-    else stage_combine_line<2, NL, KT>(cb, k, o, dt, kn);
 }
 
 // k = M^-1 r for every element and component.  Elements whose mass matrix is
@@ -228,7 +175,7 @@ __global__ __launch_bounds__(TPB) void minv_kernel(DevSpace S, const double* __r
 #pragma unroll
     for (int v = 0; v < M; ++v) kn[v] = sg ? (KT)(1e-8 * r[o + v]) : (KT)cur[(le * NB + kk) * M + v];
     if (cb.out) {
-        const double dt = (cb.stp && cb.stp->done) ? 0.0 : (cb.dte ? cb.dte[e] : *cb.dtp);
+        const double dt = stage_dt(cb, e);
 #pragma unroll
         for (int v = 0; v < M; ++v) {
             sum[v] += cb.cn * (double)kn[v];
@@ -431,7 +378,7 @@ __global__ __launch_bounds__((MinvLines<P, M, KT>::BLOCK), (MinvLines<P, M, KT>:
         return;
     }
     // (the last stage updates the state in place: out is base)
-    const double dt = (cb.stp && cb.stp->done) ? 0.0 : (cb.dte ? cb.dte[e] : *cb.dtp);
+    const double dt = stage_dt(cb, e);
     stage_combine_line<N * M, KT>(cb, k, o, dt, &kn[0][0]);
 }
 
@@ -555,7 +502,7 @@ __global__ __launch_bounds__((MinvLines2<P, M>::BLOCK), (MinvLines2<P, M>::MINW)
             kn[i][v] = sg ? (KT)(1e-8 * r[o + i * M + v]) : (KT)acc;
         }
     if (cb.out) {
-        const double dt = (cb.stp && cb.stp->done) ? 0.0 : (cb.dte ? cb.dte[e] : *cb.dtp);
+        const double dt = stage_dt(cb, e);
         stage_combine_line<N * M, KT>(cb, k, o, dt, &kn[0][0]);
         return;
     }
@@ -707,19 +654,7 @@ template <class KT>
 int minv_combine_t(int ndim, int p, int neq, const DevSpace& S, const double* r, KT* k, const KT* base, int nprev,
                    const KT* const* kk, const double* c, const double* dtp, const double* dte,
                    const StepState* stp, KT* out, bool store_k, hipStream_t st) {
-    StageComb<KT> cb;
-    cb.out = out;
-    cb.base = base;
-    cb.k0 = nprev > 0 ? kk[0] : nullptr;
-    cb.k1 = nprev > 1 ? kk[1] : nullptr;
-    cb.nprev = nprev;
-    cb.c0 = nprev > 0 ? c[0] : 0.0;
-    cb.c1 = nprev > 1 ? c[1] : 0.0;
-    cb.cn = c[nprev];
-    cb.dtp = dtp;
-    cb.dte = dte;
-    cb.stp = stp;
-    cb.store_k = store_k;
+    const StageComb<KT> cb = make_stage<KT>(base, nprev, kk, c, dtp, dte, stp, out, store_k);
     return minv_dispatch(ndim, p, neq, S, r, k, st, cb);
 }
 
