@@ -68,11 +68,11 @@ def parse():
 
 def kernel_event_pass(engine, space, disc, u, r, precision, nres):
     """The per-kernel durations: nres more residuals of the same state with
-    HIP events recorded on the launch stream before and between the three
-    kernels.  Each event costs the stream a few microseconds, so the timed
-    pass that gives the throughput carries none.  Returns (summed per-kernel
-    ms [trace, flux, element], residuals profiled, ms per residual of this
-    pass)."""
+    HIP events recorded on the launch stream before, between and after its
+    launches.  Each event costs the stream a few microseconds, so the timed
+    pass that gives the throughput carries none.  Returns (summed ms of the
+    three intervals, a one-launch residual in the last, residuals profiled,
+    ms per residual of this pass)."""
     import torch
     disc.profile_begin(nres)
     start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -85,7 +85,7 @@ def kernel_event_pass(engine, space, disc, u, r, precision, nres):
     return stage_ms, ncalls, start.elapsed_time(stop) / nres
 
 
-KERNEL_KEYS = (("trace", "trace_kernel"), ("flux", "flux_kernel"), ("element", "element_kernel"))
+KERNEL_KEYS = (("residual", "wave2d_kernel"),)  # the one launch of the headline residual
 
 
 def traffic_probe(args):
@@ -367,27 +367,18 @@ def euler3d(args, n=64, order=3, nres=30, nsteps=50):
     res_ms = start.elapsed_time(stop) / nres
     stage_ms, ncalls, _ = kernel_event_pass(engine, space, disc, u, r, "fp64", nres)
     assert bool(torch.isfinite(r).all())
-    # mixed-precision residual (FP32 interpolation, fluxes and face data),
-    # with each element-kernel tile: 0-2 the VALU kernel in 256 / 128 / 64
-    # threads, 3 the kernel whose tensor contractions run on the matrix cores
+    # mixed-precision residual (FP32 fluxes)
     r32 = torch.empty_like(u)
-    per_tile = {}
-    for t in range(4):
-        disc.set_tile(t)
-        for _ in range(3):
-            engine.form_residual(space, disc, u, r32, precision="mixed")
-        torch.cuda.synchronize()
-        start.record()
-        for _ in range(nres):
-            engine.form_residual(space, disc, u, r32, precision="mixed")
-        stop.record()
-        torch.cuda.synchronize()
-        per_tile[t] = (start.elapsed_time(stop) / nres, float((r32 - r).abs().max() / r.abs().max()))
-    mixed_tile = min(per_tile, key=lambda t: per_tile[t][0])
-    disc.set_tile(mixed_tile)
+    for _ in range(3):
+        engine.form_residual(space, disc, u, r32, precision="mixed")
+    torch.cuda.synchronize()
+    start.record()
+    for _ in range(nres):
+        engine.form_residual(space, disc, u, r32, precision="mixed")
+    stop.record()
+    torch.cuda.synchronize()
+    mixed_ms, mixed_err = start.elapsed_time(stop) / nres, float((r32 - r).abs().max() / r.abs().max())
     mstage, mcalls, _ = kernel_event_pass(engine, space, disc, u, r32, "mixed", nres)
-    mixed_ms, mixed_err = per_tile[mixed_tile]
-    valu_best = min((0, 1, 2), key=lambda t: per_tile[t][0])
     # explicit steps at a fixed dt (CFL 0.2 over the element size and the
     # initial maximum wave speed |v| + c ~ 2.9 + 1.1)
     h = 40.0 / n
@@ -407,15 +398,10 @@ def euler3d(args, n=64, order=3, nres=30, nsteps=50):
     return {
         "metric": "residual GDOF/s, 3D Euler vortex (FP64, 1 GPU)", "value": round(ndof / (res_ms * 1e-3) / 1e9, 4),
         "unit": "GDOF/s", "n_gpus": 1, "ms_per_residual": round(res_ms, 4),
-        "kernels_ms": {k: round(v / ncalls, 4) for k, v in zip(("trace", "flux", "element"), stage_ms)},
+        "kernels_ms": {"residual": round(sum(stage_ms) / ncalls, 4)},
         "mixed": {"value": round(ndof / (mixed_ms * 1e-3) / 1e9, 4), "ms_per_residual": round(mixed_ms, 4),
-                  "rel_err_vs_fp64": mixed_err, "tile": mixed_tile,
-                  "kernels_ms": {k: round(v / mcalls, 4) for k, v in zip(("trace", "flux", "element"), mstage)},
-                  "element_kernel_matrix_cores": {
-                      "ms_per_residual": round(per_tile[3][0], 4), "rel_err_vs_fp64": per_tile[3][1],
-                      "instruction": "v_mfma_f32_4x4x1f32 (16 blocks of 4 x 4 per wave, one tensor line per lane)"},
-                  "element_kernel_valu_best": {"tile": valu_best, "ms_per_residual": round(per_tile[valu_best][0], 4),
-                                               "rel_err_vs_fp64": per_tile[valu_best][1]}},
+                  "rel_err_vs_fp64": mixed_err,
+                  "kernels_ms": {"residual": round(sum(mstage) / mcalls, 4)}},
         "rk3_ssp_step_ms": round(step_ms, 4), "rk3_steps_timed": nsteps, "dt": dt,
         "element_tile": {"best": tile, "ms": [round(t, 4) for t in tile_ms]},
         "higher_is_better": True, "dtype": "f64", "data": "synthetic",
@@ -650,23 +636,16 @@ def main():
     gdofs = ndof / (ms_per_step * 1e-3) / 1e9
     assert bool(torch.isfinite(r).all())
 
-    # bytes each kernel moves by its design (state, geometry, face records,
-    # the intermediate traces and face fluxes), for the per-kernel figures
+    # bytes the one launch moves by its design: state, source load, geometry,
+    # face geometry rows (each by both elements), residual; the neighbours'
+    # states come from the caches
     info = space.info
     D, nb, nfq = space.ndim, space.nbasis, space.nfqp
     E, nfi, nfb = space.nelem, info.nface_interior, info.nface_boundary
     F = nfi + nfb
-    nvert = 2 ** D
-    nv = 1 + D  # trace record: value + the element's share of the DDG gradient
-    geo_rec = 8 * (D + 2)  # normal, w sqrt(g), h per face point
-    trace_bytes = 8 * E * 2 * D * nfq * nv * neq
-    design_bytes = {
-        "trace": 8 * E * nb * neq + 8 * E * nvert * D + 4 * 2 * D * E + geo_rec * E * 2 * D * nfq + trace_bytes,
-        "flux": trace_bytes + 16 * F + geo_rec * F * nfq + 8 * nfb * nfq * neq + 8 * F * nfq * neq,
-        "element": 8 * E * nb * neq + 8 * E * nvert * D + 4 * 2 * D * E + 8 * F * nfq * neq
-                   + 8 * E * nb * neq + 8 * E * nb * neq,
-    }
-    kms = {k: stage_ms[n] / ncalls for n, k in enumerate(("trace", "flux", "element"))}
+    design_bytes = {"residual": 3 * 8 * E * nb * neq + 8 * E * 2 ** D * D + 4 * (4 * D + 1) * E
+                    + 8 * (D + 2) * F * nfq + 8 * nfb * nfq * neq}
+    kms = {"residual": sum(stage_ms) / ncalls}
     nnode = (args.n + 1) ** 2
     b_alg = workloads.residual_bytes(D, order, neq, E, nnode, F)
     res_gbs = b_alg / (ms_per_step * 1e-3) / 1e9
@@ -712,7 +691,7 @@ def main():
         "unit": "GDOF/s",
         "ms_per_step": round(mixed_ms, 6),
         "rel_err_vs_fp64": float(f"{mixed_err:.3e}"),
-        "kernels_ms": {k: round(v / mcalls, 6) for k, v in zip(("trace", "flux", "element"), mstage)},
+        "kernels_ms": {"residual": round(sum(mstage) / mcalls, 6)},
         "arithmetic": "FP32 interpolation, fluxes and face data; FP64 geometry, source load and output",
     }
 
@@ -782,12 +761,12 @@ def main():
                          "threads": [256, 128, 64]},
         "roofline": {
             "bound": "hbm",
-            "kernel": "residual = trace_kernel + flux_kernel + element_kernel_2d (3 launches, timed pass)",
+            "kernel": "wave2d_kernel (one launch per residual, timed pass)",
             "achieved": round(res_gbs, 2),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": round(res_gbs / HBM_PEAK_GBS, 5),
-            "traffic": (int(sum(traffic.values())) if traffic and len(traffic) == 3 else None),
+            "traffic": (int(sum(traffic.values())) if traffic and len(traffic) == len(KERNEL_KEYS) else None),
             "bytes_per_launch": int(b_alg),
             "bytes_formula": "2*8*m*E*nb + 8*d*N_vert + 4*2^d*E + 12*(F_i+F_b)",
             "traffic_source": traffic_info if traffic is None else

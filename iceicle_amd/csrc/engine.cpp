@@ -517,6 +517,12 @@ static int space_create(const ice_mesh_desc* mds, int nmesh, const ice_space_des
             if (fnr != (fnl + D) % (2 * D) || std::memcmp(tl, tr, s->nfq) != 0)
                 throw ice::Error{ICE_ERR_UNSUPPORTED, "elements of a structured mesh are not aligned"};
         }
+        // (and a face's own order of its points mirrors the tensor order, its own inverse)
+        for (int j = 0; j < 2 * D; ++j)
+            for (int q = 0; q < s->nfq; ++q) {
+                const signed char* t = &s->ftens[(size_t)j * no * s->nfq];
+                if (t[t[q]] != q) throw ice::Error{ICE_ERR_UNSUPPORTED, "face point order is not a mirror"};
+            }
         for (int f = 0; f < nfi; ++f) {
             const int4 r = s->fint[f];
             const int fnl = r.z & 7, fnr = (r.z >> 3) & 7, orient = (r.z >> 6) & 7;
@@ -590,6 +596,7 @@ static int space_create(const ice_mesh_desc* mds, int nmesh, const ice_space_des
         dv.nfb = nfb;
         dv.norient = no;
         for (int d = 0; d < 3; ++d) dv.period[d] = m.period[d];
+        for (int d = 0; d < 3; ++d) dv.nel[d] = m.nel[d];
         dv.X = (const double*)s->dmem[0];
         dv.fint = (const int4*)s->dmem[1];
         dv.fbdy = (const int4*)s->dmem[2];
@@ -872,9 +879,7 @@ int ice_disc_autotune(ice_disc* d, const double* u, double* r, int reps, int* be
     // the bytes, so the fastest shape can differ)
     for (int prec = 0; prec < 2 && rc == ICE_OK; ++prec) {
         double tbest = 1e300;
-        // tile 3 (matrix cores) exists for the mixed residual of 3D P3 Euler only
-        const bool mfma = prec == 1 && s->ndim == 3 && s->p == 3 && d->prm.flux == ICE_FLUX_EULER;
-        for (int tile = 0; tile < (mfma ? 4 : 3) && rc == ICE_OK; ++tile) {
+        for (int tile = 0; tile < 3 && rc == ICE_OK; ++tile) {
             d->dd.tile = tile;
             d->dd.tile_mixed = tile;
             auto once = [&]() {
@@ -1233,17 +1238,23 @@ int step_once(ice_stepper* S, double* u, hipStream_t st) {
             axpy(1.0 / 6.0, k1, u);
             axpy(1.0 / 6.0, k1, u);
             axpy(2.0 / 3.0, k1, u);
-        } else if (ice::wave2d_covers(sp->ndim, sp->p, d->dd)) {
-            // a launch per stage: residual, increment and combination; no
-            // stage may write the state it reads, so the third's is in k3
-            auto stage = [&](const double* x, double* k, int nprev, const double* c, double* out, bool store_k) {
-                const double* kk[2] = {k1, k2};
-                const auto cb = ice::make_stage<double>(u, nprev, kk, c, dt, S->dte, S->st, out, store_k);
-                rc |= ice::residual_stage(sp->ndim, sp->p, d->prm.flux, sp->dev, d->ph, d->dd, x, k, cb, st);
+        } else if (ice::wave_covers(sp->ndim, sp->p, d->prm.flux, d->dd)) {
+            // a launch per stage: residual, inverse mass and combination in
+            // its increment-free form; no stage may write the state it reads
+            auto stage = [&](const double* x, double cx, double* out) {
+                ice::StageComb<double> cb;
+                cb.out = out;
+                cb.base = u;
+                cb.dtp = dt;
+                cb.dte = S->dte;
+                cb.stp = S->st;
+                cb.first = x == u;
+                cb.cx = cx;
+                rc |= ice::residual_stage(sp->ndim, sp->p, d->prm.flux, sp->dev, d->ph, d->dd, x, nullptr, cb, st);
             };
-            stage(u, k1, 0, C1, us, true);
-            stage(us, k2, 1, C2, k3, true);
-            stage(k3, res, 2, C3, u, false);
+            stage(u, 1.0, us);
+            stage(us, 0.25, k3);
+            stage(k3, 2.0 / 3.0, u);
         } else {
             // ssp_rk3.hpp:164-190; each stage's increment and combination
             // u1 = u + dt k1, u2 = u + dt (k1 + k2)/4, u = u + dt (k1/6 + k2/6 + 2 k3/3)
@@ -1306,7 +1317,7 @@ int step_once(ice_stepper* S, float* u, hipStream_t st) {
     };
     const float* kk[2] = {k1, k2};
     rc |= ice::launch_step_begin(S->st, d->d_wave, S->ctl, st);
-    if (S->desc.kind == ICE_STEP_RK3_SSP && ice::wave2d_covers(sp->ndim, sp->p, d->dd)) {
+    if (S->desc.kind == ICE_STEP_RK3_SSP && ice::wave_covers(sp->ndim, sp->p, d->prm.flux, d->dd)) {
         auto stage = [&](const float* x, float* k, int nprev, const double* c, float* out, bool store_k) {
             const auto cb = ice::make_stage<float>(u, nprev, kk, c, dt, S->dte, S->st, out, store_k);
             rc |= ice::residual_stage(sp->ndim, sp->p, d->prm.flux, sp->dev, d->ph, d->dd, x, k, cb, st);

@@ -19,6 +19,7 @@ struct DevSpace {
     int nfb;                 // boundary faces, Q rows [nfi, nfi + nfb)
     int norient;             // orientation codes per face number in fpt
     double period[3];
+    int nel[3];              // elements per direction of a single structured mesh (0: several meshes)
     const double* X;         // [nelem][2^ndim][ndim] element vertex coordinates
     const int4* fint;        // {elemL, elemR, info, 0}
     const int4* fbdy;        // {elemL, info, bcflag, 0}
@@ -120,9 +121,13 @@ int launch_widen(size_t n, const float* x, double* y, hipStream_t st);  // y = (
 int launch_step_begin(StepState* s, unsigned long long* wave, const StepControl& c, hipStream_t st);
 int launch_step_end(StepState* s, hipStream_t st);
 
-// One-launch 2D residual (residual_wave2d.h); with cb.out the stage form:
-// K = M^-1 R(U) and the stage combination, U not aliasing cb.out.
-inline bool wave2d_covers(int ndim, int p, const DiscDev& dd) { return ndim == 2 && p <= 3 && !dd.Pic; }
+// One-launch residuals (residual_wave2d.h, residual_wave3d.h): 2D P1-P3
+// without DDGIC vectors, 3D Euler P2 and P3.
+inline bool wave_covers(int ndim, int p, int flux, const DiscDev& dd) {
+    return (ndim == 2 && p <= 3 && !dd.Pic) || (ndim == 3 && flux == ICE_FLUX_EULER && (p == 2 || p == 3));
+}
+// Their stage form: K = M^-1 R(U) and the stage combination cb, U not
+// aliasing cb.out.
 int residual_stage(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                    const double* U, double* K, const StageComb<double>& cb, hipStream_t st);
 int residual_stage(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,

@@ -482,106 +482,6 @@ __global__ __launch_bounds__(TPB, ICE_TRACE_MINW) void trace_kernel(DevSpace S, 
     for (int idx = threadIdx.x; idx < ne * TPE * NV * M; idx += blockDim.x) dst[idx] = sOut[idx];
 }
 
-// 3D P3 traces of fluxes without a gradient, two points of a face row per
-// thread: along the face normal only the face's N^2 nodes contribute, and the
-// contraction along the face's first tangential axis, t[ib] = sum_ia
-// l_ia(s_a) U[ia][ib], is shared by the points of a row (canonical face
-// points run row by row).  Per point: 40 LDS reads and 50 FMA per variable
-// set instead of 80 and 80 with one point per thread.  The element tile's
-// coefficients and its trace records share one LDS buffer.
-template <class PH, int EPB, class UT = double>
-__global__ __launch_bounds__(((EPB * 48 + 63) / 64) * 64) void trace_kernel_rows(DevSpace S, typename PH::Params ph,
-                                                                                 const UT* __restrict__ U,
-                                                                                 typename PH::real* __restrict__ T) {
-    using VT = typename PH::real;
-    constexpr int D = 3, N = 4, NN = 16, NB = 64, NFQ = 16;
-    constexpr int M = PH::M;
-    constexpr int TPE = 2 * D * NN / 2;  // threads per element: two points each
-    constexpr int PTE = 2 * D * NFQ;     // trace points per element
-    static_assert(!TraceRec<PH, D>::NEED_GRAD, "fluxes without a gradient");
-    constexpr int BUF = (EPB * PTE * M > EPB * NB * M) ? EPB * PTE * M : EPB * NB * M;
-    __shared__ VT sbuf[BUF];
-    __shared__ VT sL[(N + 2) * N];
-    const int e0 = blockIdx.x * EPB;
-    const int le = threadIdx.x / TPE;
-    const int t = threadIdx.x - le * TPE;
-    const int e = e0 + le;
-    const bool active = threadIdx.x < EPB * TPE && e < S.nelem;
-    const int j = t / (NN / 2), rem = t - j * (NN / 2);
-    const int s0 = rem / 2, s1 = 2 * (rem - s0 * 2);  // canonical points q0 = s0 N + s1, q0 + 1
-    {
-        const size_t base = (size_t)e0 * NB * M;
-        const size_t total = (size_t)S.nelem * NB * M;
-        for (int idx = threadIdx.x; idx < EPB * NB * M; idx += blockDim.x)
-            sbuf[idx] = coef_stage<VT, NB, M, UT>(U, base, total, idx);
-        const VT* tv = tab_of<VT>(S) + (N + 2);
-        for (int idx = threadIdx.x; idx < (N + 2) * N; idx += blockDim.x) sL[idx] = tv[idx];
-    }
-    int pa[D] = {}, pb[D] = {};
-    if (active) {
-        const signed char* fp = S.fpt + ((size_t)(j * S.norient + 0) * NFQ + s0 * N + s1) * D;
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            pa[d] = fp[d];
-            pb[d] = fp[D + d];
-        }
-    }
-    __syncthreads();
-    VT out[2][M];
-    if (active) {
-        const int kn = j % D;
-        const int inode = (j < D) ? 0 : N - 1;
-        const VT* Ue = sbuf + (size_t)le * NB * M;
-        auto row = [&](auto KN) {
-            constexpr int K = decltype(KN)::value;
-            constexpr int TA = (K == 0) ? 1 : 0, TB = (K == 2) ? 1 : 2;
-            constexpr int SK = Pow<N, 2 - K>::value, SA = Pow<N, 2 - TA>::value, SB = Pow<N, 2 - TB>::value;
-            const VT en = sL[pa[K] * N + inode];
-            VT la[N];
-#pragma unroll
-            for (int i = 0; i < N; ++i) la[i] = sL[pa[TA] * N + i] * en;
-            const VT* Ub = Ue + inode * SK * M;
-#pragma unroll
-            for (int v = 0; v < M; ++v) out[0][v] = out[1][v] = VT(0);
-            // one tangential column per pass (unrolled, the face's 80 values
-            // would be loaded at once and halve the occupancy)
-#pragma unroll 1
-            for (int ib = 0; ib < N; ++ib) {
-                const VT* Uc = Ub + ib * SB * M;
-                VT tv[M];
-#pragma unroll
-                for (int v = 0; v < M; ++v) tv[v] = VT(0);
-#pragma unroll
-                for (int ia = 0; ia < N; ++ia)
-#pragma unroll
-                    for (int v = 0; v < M; ++v) tv[v] += Uc[ia * SA * M + v] * la[ia];
-                const VT b0 = sL[pa[TB] * N + ib], b1 = sL[pb[TB] * N + ib];
-#pragma unroll
-                for (int v = 0; v < M; ++v) {
-                    out[0][v] += tv[v] * b0;
-                    out[1][v] += tv[v] * b1;
-                }
-            }
-        };
-        if (kn == 0) row(std::integral_constant<int, 0>{});
-        else if (kn == 1) row(std::integral_constant<int, 1>{});
-        else row(std::integral_constant<int, 2>{});
-    }
-    __syncthreads();  // the coefficients are read: the buffer takes the records
-    if (active) {
-        VT* o = sbuf + ((size_t)le * PTE + j * NFQ + s0 * N + s1) * M;
-#pragma unroll
-        for (int k = 0; k < 2; ++k)
-#pragma unroll
-            for (int v = 0; v < M; ++v) o[k * M + v] = out[k][v];
-    }
-    __syncthreads();
-    // records of elements e0 .. e0 + ne - 1 are one contiguous range of T
-    const int ne = min(EPB, S.nelem - e0);
-    VT* dst = T + (size_t)e0 * PTE * M;
-    for (int idx = threadIdx.x; idx < ne * PTE * M; idx += blockDim.x) dst[idx] = sbuf[idx];
-}
-
 // Numerical flux (and DDGIC lifting vector) at point q of interior face f
 // from the two trace records of the point (left element tL, right tR), ph
 // the left element's flux parameters.
@@ -838,10 +738,8 @@ struct ElemTile {
     static constexpr int NT = EPB * NB;
     static constexpr int BLOCK = ((NT + 63) / 64) * 64;
 };
-// workgroup size targets selected by DiscDev::tile (TILE_MFMA: the matrix-core
-// 3D P3 kernel of the mixed residual where it applies, else the default tile)
+// workgroup size targets selected by DiscDev::tile
 constexpr int tile_tpb(int tile) { return tile == 1 ? 128 : tile == 2 ? 64 : 256; }
-constexpr int TILE_MFMA = 3;
 
 template <int D, int P, class PH>
 __global__ __launch_bounds__(256) void element_kernel(DevSpace S, PhysParams ph0, const double* __restrict__ emu,
@@ -1893,310 +1791,6 @@ __global__ __launch_bounds__((Elem3Tile<P, TPB>::BLOCK), ICE_ELEM3_MINW) void el
     for (int v = 0; v < M; ++v) Re[v] = r[v];
 }
 
-// ---- 3D P3 element kernel on the matrix cores (FP32, fluxes without a
-// gradient) ------------------------------------------------------------------
-// The sum-factorised contractions of element_kernel_3d are 4 x 4 operators
-// applied along one axis of each element's [var][4][4][4] tensors.  Here
-// one lane owns one tensor line (4 entries along the contracted axis) and
-// the wave applies the operator to 64 lines at once with
-// v_mfma_f32_4x4x1f32 (16 blocks of 4 x 4 outer products): lane 4b + r
-// supplies operator row r, lane l its line's entry c, and after the four
-// K = 1 steps lane l holds its line's 4 outputs (register r = output r).
-// Each phase writes its outputs rotated, [ev][r][x][y] for the input line
-// [ev][x][y][:], so the next phase's contraction axis is again contiguous
-// (one 16-byte LDS read per line) and three rotations restore the natural
-// point order.  Interpolation to the quadrature points (3 phases), the flux
-// at each point (one thread per point, FP64 geometry), the test
-// contractions (2a: three arrays, 2b: two with the sum of the second and
-// third, 2c: one), then per node the source load, the face lifting and the
-// FP64 store, as element_kernel_3d.
-typedef float ice_floatx4 __attribute__((ext_vector_type(4)));
-
-template <int M>
-struct Elem3Mfma {
-    static constexpr int EPB = 4;                          // elements per workgroup
-    static constexpr int LINES = EPB * M * 16;             // tensor lines per array
-    static constexpr int NWAVE = (LINES / 64 > EPB) ? LINES / 64 : EPB;  // line waves, or a wave per element
-    static constexpr int BLOCK = 64 * NWAVE;
-    // LDS stride of one [ev] tensor: a multiple of 16 floats that is 16 mod
-    // 64, so the rotated stores of the 4 tensors a wave covers fall on
-    // distinct banks
-    static constexpr int EVS = 80;
-    static constexpr int ARR = EPB * M * EVS;              // one array of the workgroup
-};
-
-// 4 x 4 contraction of the lane's line x: returns out[r] = sum_c A[r][c] x[c]
-// when lane l passes a[c] = A[l % 4][c]
-__device__ __forceinline__ ice_floatx4 mfma_line(const float (&a)[4], const float (&x)[4], ice_floatx4 acc) {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) acc = __builtin_amdgcn_mfma_f32_4x4x1f32(a[c], x[c], acc, 0, 0, 0);
-    return acc;
-}
-
-// line L = (ev, x, y) of an array with [ev] stride EVS: its 4 entries start at
-__device__ __forceinline__ int mfma_line_base(int L, int evs) { return (L >> 4) * evs + (L & 15) * 4; }
-// rotated output slot r of line L: [ev][r][x][y]
-__device__ __forceinline__ int mfma_rot_slot(int L, int r, int evs) { return (L >> 4) * evs + r * 16 + (L & 15); }
-
-template <class PH, class UT = double>
-__global__ __launch_bounds__(Elem3Mfma<PH::M>::BLOCK) void element_kernel_3d_mfma(
-    DevSpace S, typename PH::Params ph0, const double* __restrict__ emu, const double* __restrict__ srcload,
-    const UT* __restrict__ U, const float* __restrict__ Q, double* __restrict__ R,
-    unsigned long long* __restrict__ wave, double* __restrict__ wave_part) {
-    constexpr int D = 3, N = 4, NN = 16, NB = 64, NFQ = 16;
-    constexpr int M = PH::M;
-    using TL = Elem3Mfma<M>;
-    constexpr int EPB = TL::EPB, LINES = TL::LINES, EVS = TL::EVS, ARR = TL::ARR, BLOCK = TL::BLOCK;
-    constexpr int NV = 1 << D;
-    constexpr int NT2 = (N + 2) * N;
-    constexpr int LIFT = 2 * D * NFQ * M;
-    static_assert(!TraceRec<PH, D>::NEED_GRAD, "fluxes without a gradient");
-    static_assert((LINES % 64) == 0, "whole waves of tensor lines");
-    __shared__ __align__(16) float s0[3 * ARR];
-    __shared__ __align__(16) float s1[3 * ARR];
-    __shared__ float sQ[EPB * LIFT];
-    __shared__ float sL[2 * NT2];
-    __shared__ double sLd[NT2];
-    __shared__ double sX[EPB * NV * D];
-    __shared__ int sEF[EPB * 2 * D];
-    __shared__ signed char sFT[2 * D * 8 * NFQ];
-    __shared__ double red[2 * (BLOCK / 64)];
-    __shared__ double sU0[EPB * M];  // each element's first coefficients (coefficients staged as U_i - U_0)
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wv = tid >> 6;
-    const int e0 = blockIdx.x * EPB;
-    // prologue: coefficients as [ev][node] (ev = element * M + var), tables,
-    // vertices, face slots
-    {
-        const size_t base = (size_t)e0 * NB * M, total = (size_t)S.nelem * NB * M;
-        for (int idx = tid; idx < EPB * NB * M; idx += BLOCK) {
-            const int l = idx / (NB * M), rem = idx - l * (NB * M);
-            const int node = rem / M, v = rem - node * M;
-            s0[(l * M + v) * EVS + node] = coef_stage<float, NB, M, UT>(U, base, total, idx);
-        }
-        for (int idx = tid; idx < EPB * M; idx += BLOCK) {
-            const size_t g = base + (size_t)(idx / M) * NB * M + idx % M;
-            sU0[idx] = g < total ? (double)U[g] : 0.0;
-        }
-        const size_t xb = (size_t)e0 * NV * D, xt = (size_t)S.nelem * NV * D;
-        for (int idx = tid; idx < EPB * NV * D; idx += BLOCK) sX[idx] = (xb + idx < xt) ? S.X[xb + idx] : 0.0;
-        const size_t fb = (size_t)e0 * 2 * D, ft = (size_t)S.nelem * 2 * D;
-        for (int idx = tid; idx < EPB * 2 * D; idx += BLOCK) sEF[idx] = (fb + idx < ft) ? S.efaces[fb + idx] : -1;
-        for (int idx = tid; idx < 2 * NT2; idx += BLOCK) sL[idx] = S.tabf[(N + 2) + idx];
-        for (int idx = tid; idx < NT2; idx += BLOCK) sLd[idx] = S.tab[(N + 2) + idx];
-        for (int idx = tid; idx < 2 * D * 8 * NFQ && idx < 2 * D * S.norient * NFQ; idx += BLOCK)
-            sFT[idx] = S.ftens[idx];
-    }
-    __syncthreads();
-    // face fluxes in the face's tensor order (as element_kernel_3d): loaded
-    // into registers now, stored to LDS after the first contraction phase,
-    // so their latency overlaps it
-    constexpr int QIT = (EPB * LIFT + BLOCK - 1) / BLOCK;
-    float qv[QIT];
-    int qdst[QIT];
-#pragma unroll
-    for (int it = 0; it < QIT; ++it) {
-        const int idx = tid + it * BLOCK;
-        const int l = idx / LIFT, rem = idx - l * LIFT;
-        const int j = rem / (NFQ * M), w = rem - j * (NFQ * M);
-        const int fq = w / M, v = w - fq * M;
-        const int ef = (idx < EPB * LIFT) ? sEF[l * 2 * D + j] : -1;  // faces without a slot are not lifted
-        qv[it] = (ef >= 0) ? Q[(size_t)(ef >> 4) * NFQ * M + w] : 0.f;
-        qdst[it] = (ef >= 0) ? l * LIFT + (j * NFQ + sFT[(j * S.norient + (ef & 7)) * NFQ + fq]) * M + v : -1;
-    }
-    // per-lane operator rows: interpolation a[c] = L0[point r][basis c],
-    // test contractions with L0^T and L1^T: a[c] = L[point c][basis r]
-    const int r4 = lane & 3;
-    float aI[4], aT0[4], aT1[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        aI[c] = sL[r4 * N + c];
-        aT0[c] = sL[c * N + r4];
-        aT1[c] = sL[NT2 + c * N + r4];
-    }
-    // one rotation pass: lines of `in` (any count, uniform per wave) -> `out`
-    auto rotate = [&](const float* in, float* out, const float (&a)[4]) {
-#pragma unroll 1
-        for (int g = wv; g < LINES / 64; g += BLOCK / 64) {
-            const int L = g * 64 + lane;
-            const float4 xv = *reinterpret_cast<const float4*>(in + mfma_line_base(L, EVS));
-            const float x[4] = {xv.x, xv.y, xv.z, xv.w};
-            ice_floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-            acc = mfma_line(a, x, acc);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) out[mfma_rot_slot(L, r, EVS)] = acc[r];
-        }
-    };
-    // 1a, 1b, 1c: u at the quadrature points, natural order, in s1[0]
-    rotate(s0, s1, aI);
-#pragma unroll
-    for (int it = 0; it < QIT; ++it)
-        if (qdst[it] >= 0) sQ[qdst[it]] = qv[it];
-    __syncthreads();
-    rotate(s1, s0, aI);
-    __syncthreads();
-    rotate(s0, s1, aI);
-    __syncthreads();
-    // flux at each point: contravariant fluxes G_a = F . adj(J)[a] detc w / det into s0[a]
-    const double* xs = S.tab;
-    const double* wgl = S.tab + (N + 2) + 3 * (N + 2) * N;
-    double lam_w = 0.0, vis_w = 0.0;
-    for (int t = tid; t < EPB * NB; t += BLOCK) {
-        const int l = t / NB, k = t - l * NB;
-        const int e = e0 + l;
-        if (e >= S.nelem) continue;
-        const int k0 = k / NN, k1 = (k / N) % N, k2 = k % N;
-        const typename PH::Params ph = local_params(ph0, emu, e);
-        double X[NV][D];
-#pragma unroll
-        for (int i = 0; i < NV; ++i)
-#pragma unroll
-            for (int d = 0; d < D; ++d) X[i][d] = sX[(l * NV + i) * D + d];
-        const double xi[D] = {xs[k0], xs[k1], xs[k2]};
-        const double wq = wgl[k0] * wgl[k1] * wgl[k2];
-        double J[D][D], Hm[D][D][D], A[D][D];
-        q1_map<D>(X, xi, nullptr, J, Hm);
-        const double det = det_adj<D>(J, A);
-        const double detc = fmax(0.0, det);
-        const double detg = (det == 0.0) ? 1.0 : det;
-        const double fac = detc * wq / detg;
-        float u[M], gx[M * D] = {}, F[M * D];
-#pragma unroll
-        for (int v = 0; v < M; ++v) u[v] = (float)((double)s1[(l * M + v) * EVS + k] + sU0[l * M + v]);
-        PH::flux(ph, u, gx, F);
-        if (wave) {
-            lam_w = fmax(lam_w, (double)PH::wave_speed(ph, u));
-            vis_w = fmax(vis_w, (double)PH::visc_at(ph, u));
-            if (e == S.nelem - 1 && k == NB - 1) wave[1] = (unsigned long long)__double_as_longlong((double)PH::wave_speed(ph, u));
-        }
-        float ga[D][D];
-#pragma unroll
-        for (int a = 0; a < D; ++a)
-#pragma unroll
-            for (int j = 0; j < D; ++j) ga[a][j] = (float)(A[a][j] * fac);
-#pragma unroll
-        for (int a = 0; a < D; ++a)
-#pragma unroll
-            for (int v = 0; v < M; ++v)
-                s0[a * ARR + (l * M + v) * EVS + k] = F[v * D + 0] * ga[a][0] + F[v * D + 1] * ga[a][1] +
-                                                     F[v * D + 2] * ga[a][2];
-    }
-    if (wave) {
-        for (int off = 32; off > 0; off >>= 1) {
-            lam_w = fmax(lam_w, __shfl_xor(lam_w, off));
-            vis_w = fmax(vis_w, __shfl_xor(vis_w, off));
-        }
-        if (lane == 0) {
-            red[2 * wv] = lam_w;
-            red[2 * wv + 1] = vis_w;
-        }
-    }
-    __syncthreads();
-    if (wave && tid == 0) {
-        double a = 0.0, b = 0.0;
-        for (int w = 0; w < BLOCK / 64; ++w) { a = fmax(a, red[2 * w]); b = fmax(b, red[2 * w + 1]); }
-        wave_part[2 * blockIdx.x] = a;
-        wave_part[2 * blockIdx.x + 1] = b;
-    }
-    // 2a: contract q2 of G0, G1 (values) and G2 (derivatives) -> s1[a]
-#pragma unroll 1
-    for (int g = wv; g < 3 * LINES / 64; g += BLOCK / 64) {
-        const int a = g / (LINES / 64), L = (g - a * (LINES / 64)) * 64 + lane;
-        const float4 xv = *reinterpret_cast<const float4*>(s0 + a * ARR + mfma_line_base(L, EVS));
-        const float x[4] = {xv.x, xv.y, xv.z, xv.w};
-        ice_floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = (a == 2) ? mfma_line(aT1, x, acc) : mfma_line(aT0, x, acc);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s1[a * ARR + mfma_rot_slot(L, r, EVS)] = acc[r];
-    }
-    __syncthreads();
-    // 2b: contract q1: T0 = L0^T G0' -> s0[0]; T12 = L1^T G1' + L0^T G2' -> s0[1]
-#pragma unroll 1
-    for (int g = wv; g < 2 * LINES / 64; g += BLOCK / 64) {
-        const int o = g / (LINES / 64), L = (g - o * (LINES / 64)) * 64 + lane;
-        ice_floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-        const float4 xv = *reinterpret_cast<const float4*>(s1 + o * ARR + mfma_line_base(L, EVS));
-        const float x[4] = {xv.x, xv.y, xv.z, xv.w};
-        if (o == 0) {
-            acc = mfma_line(aT0, x, acc);
-        } else {
-            acc = mfma_line(aT1, x, acc);
-            const float4 yv = *reinterpret_cast<const float4*>(s1 + 2 * ARR + mfma_line_base(L, EVS));
-            const float y[4] = {yv.x, yv.y, yv.z, yv.w};
-            acc = mfma_line(aT0, y, acc);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s0[o * ARR + mfma_rot_slot(L, r, EVS)] = acc[r];
-    }
-    __syncthreads();
-    // 2c: contract q0: R = L1^T T0' + L0^T T12' -> s1[0], natural node order
-#pragma unroll 1
-    for (int g = wv; g < LINES / 64; g += BLOCK / 64) {
-        const int L = g * 64 + lane;
-        const float4 xv = *reinterpret_cast<const float4*>(s0 + mfma_line_base(L, EVS));
-        const float4 yv = *reinterpret_cast<const float4*>(s0 + ARR + mfma_line_base(L, EVS));
-        const float x[4] = {xv.x, xv.y, xv.z, xv.w}, y[4] = {yv.x, yv.y, yv.z, yv.w};
-        ice_floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = mfma_line(aT1, x, acc);
-        acc = mfma_line(aT0, y, acc);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s1[mfma_rot_slot(L, r, EVS)] = acc[r];
-    }
-    __syncthreads();
-    // per node: volume term, source load, lifting, FP64 store (element_kernel_3d)
-    for (int t = tid; t < EPB * NB; t += BLOCK) {
-        const int l = t / NB, k = t - l * NB;
-        const int e = e0 + l;
-        if (e >= S.nelem) continue;
-        const int k0 = k / NN, k1 = (k / N) % N, k2 = k % N;
-        double r[M];
-#pragma unroll
-        for (int v = 0; v < M; ++v) r[v] = (double)s1[(l * M + v) * EVS + k];
-        if (srcload) {
-            const double* sl = srcload + ((size_t)e * NB + k) * M;
-#pragma unroll
-            for (int v = 0; v < M; ++v) r[v] -= sl[v];
-        }
-        const int kd[D] = {k0, k1, k2};
-        unsigned mask = 0;
-#pragma unroll
-        for (int j = 0; j < 2 * D; ++j)
-            if (kd[j % D] == ((j < D) ? 0 : N - 1)) mask |= 1u << j;
-        while (mask) {
-            const int j = __builtin_ctz(mask);
-            mask &= mask - 1;
-            const int ef = sEF[l * 2 * D + j];
-            if (ef < 0) continue;
-            const int kn = j % D;
-            const int sa = (kn == 0) ? k1 : k0, sb = (kn == 2) ? k1 : k2;
-            const double en = sLd[((j < D) ? N : N + 1) * N + kd[kn]];
-            const double sgn = ((ef >> 3) & 1) ? -en : en;
-            double la[N], lb[N];
-#pragma unroll
-            for (int p = 0; p < N; ++p) {
-                la[p] = sLd[p * N + sa];
-                lb[p] = sLd[p * N + sb];
-            }
-            const float* Qf = sQ + l * LIFT + j * NFQ * M;
-#pragma unroll
-            for (int v = 0; v < M; ++v) {
-                double acc = 0.0;
-#pragma unroll
-                for (int pa = 0; pa < N; ++pa) {
-                    double tt = 0.0;
-#pragma unroll
-                    for (int pb = 0; pb < N; ++pb) tt += (double)Qf[(pa * N + pb) * M + v] * lb[pb];
-                    acc += tt * la[pa];
-                }
-                r[v] += sgn * acc;
-            }
-        }
-        double* Re = R + ((size_t)e * NB + k) * M;
-#pragma unroll
-        for (int v = 0; v < M; ++v) Re[v] = r[v];
-    }
-}
-
 // Fold the per-block maxima of one residual into the running maxima
 // (lambda_max of BurgersFlux never resets, burgers.hpp:89; visc_max, navier_stokes.hpp:964-966).
 __global__ void wave_reduce_kernel(const double* __restrict__ part, int nblk, unsigned long long* __restrict__ wave) {
@@ -2504,19 +2098,14 @@ int launch_residual(const DevSpace& S, const typename PH::Params& ph, const Disc
     if (ev) (void)hipEventRecord(ev[0], st);
     const int nbi = (int)(((long)S.nfi * NFQ + 255) / 256);
     const int nbb = (int)(((long)S.nfb * NFQ + 255) / 256);
-    if constexpr (D == 3 && P == 3 && !TraceRec<PH, D>::NEED_GRAD) {
-        constexpr int EPB = 4;  // 192 threads
-        trace_kernel_rows<PH, EPB, UT><<<(S.nelem + EPB - 1) / EPB, ((EPB * 48 + 63) / 64) * 64, 0, st>>>(S, ph, U, T);
-    } else {
-        constexpr int TPE = 2 * D * NFQ;
-        // whole elements per workgroup, rounded up to whole waves only once:
-        // a wave that would hold no trace point is not launched (3D P3:
-        // 2 x 96 points in 192 threads rather than 256)
-        constexpr int EPW = (TPE <= ICE_TRACE_TPB) ? ICE_TRACE_TPB / TPE : 1;
-        constexpr int TTPB = ((EPW * TPE + 63) / 64) * 64;
-        constexpr int EPB = TTPB / TPE;
-        trace_kernel<D, P, PH, TTPB, UT><<<(S.nelem + EPB - 1) / EPB, TTPB, 0, st>>>(S, ph, U, T);
-    }
+    constexpr int TPE = 2 * D * NFQ;
+    // whole elements per workgroup, rounded up to whole waves only once:
+    // a wave that would hold no trace point is not launched (3D P3:
+    // 2 x 96 points in 192 threads rather than 256)
+    constexpr int EPW = (TPE <= ICE_TRACE_TPB) ? ICE_TRACE_TPB / TPE : 1;
+    constexpr int TTPB = ((EPW * TPE + 63) / 64) * 64;
+    constexpr int EPB = TTPB / TPE;
+    trace_kernel<D, P, PH, TTPB, UT><<<(S.nelem + EPB - 1) / EPB, TTPB, 0, st>>>(S, ph, U, T);
     if (ev) (void)hipEventRecord(ev[1], st);
     if (nbb > 0)
         flux_kernel<D, P, PH, true, UT><<<nbi + nbb, 256, 0, st>>>(S, ph, d, T, nbi, U);
@@ -2540,18 +2129,6 @@ int launch_residual(const DevSpace& S, const typename PH::Params& ph, const Disc
                     d.wave, d.wave_part);
         };
         const int tile = std::is_same<VT, double>::value ? d.tile : d.tile_mixed;
-        if constexpr (D == 3 && P == 3 && std::is_same<VT, float>::value && !TraceRec<PH, D>::NEED_GRAD &&
-                      !PH::HAS_HOMOGENEITY) {
-            if (tile == TILE_MFMA) {
-                using TM = Elem3Mfma<PH::M>;
-                nblk = (S.nelem + TM::EPB - 1) / TM::EPB;
-                element_kernel_3d_mfma<PH, UT><<<nblk, TM::BLOCK, 0, st>>>(
-                    S, ph, d.emu, d.srcload, U, reinterpret_cast<const float*>(d.Q), R, d.wave, d.wave_part);
-                if (d.wave) wave_reduce_kernel<<<1, 256, 0, st>>>(d.wave_part, nblk, d.wave);
-                if (ev) (void)hipEventRecord(ev[3], st);
-                return (int)hipGetLastError();
-            }
-        }
         switch (tile) {
         case 1: go(std::integral_constant<int, tile_tpb(1)>{}); break;
         case 2: go(std::integral_constant<int, tile_tpb(2)>{}); break;
@@ -2569,21 +2146,23 @@ int launch_residual(const DevSpace& S, const typename PH::Params& ph, const Disc
     return (int)hipGetLastError();
 }
 
-// One-launch 2D residuals, one translation unit per flux family
-#define ICE_WAVE2D_DECL(F)                                                                                         \
+// One-launch residuals, one translation unit per dimension and flux family
+#define ICE_WAVE_DECL(F)                                                                                         \
     int F(int p, const DevSpace& S, const PhysT<double>& ph, const DiscDev& dd, const double* U, double* R,        \
           double* K, const StageComb<double>& cb, hipStream_t st);                                                 \
     int F(int p, const DevSpace& S, const PhysT<float>& ph, const DiscDev& dd, const double* U, double* R,         \
           hipStream_t st);                                                                                         \
     int F(int p, const DevSpace& S, const PhysT<float>& ph, const DiscDev& dd, const float* U, double* R, float* K, \
           const StageComb<float>& cb, hipStream_t st);
-ICE_WAVE2D_DECL(wave2d_burgers)
-ICE_WAVE2D_DECL(wave2d_ns)
-ICE_WAVE2D_DECL(wave2d_euler)
-#undef ICE_WAVE2D_DECL
+ICE_WAVE_DECL(wave2d_burgers)
+ICE_WAVE_DECL(wave2d_ns)
+ICE_WAVE_DECL(wave2d_euler)
+ICE_WAVE_DECL(wave3d_euler)
+#undef ICE_WAVE_DECL
 
 template <class R, class... A>
-int wave2d_flux(int flux, int p, const DevSpace& S, const PhysT<R>& ph, const DiscDev& dd, A... a) {
+int wave_residual(int flux, int p, const DevSpace& S, const PhysT<R>& ph, const DiscDev& dd, A... a) {
+    if (S.ndim == 3) return wave3d_euler(p, S, ph, dd, a...);
     if (flux == ICE_FLUX_BURGERS) return wave2d_burgers(p, S, ph, dd, a...);
     if (flux == ICE_FLUX_NAVIER_STOKES) return wave2d_ns(p, S, ph, dd, a...);
     if (flux == ICE_FLUX_EULER) return wave2d_euler(p, S, ph, dd, a...);
@@ -2601,26 +2180,28 @@ int profiled(hipEvent_t* ev, hipStream_t st, F launch) {
 
 int residual_stage(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                    const double* U, double* K, const StageComb<double>& cb, hipStream_t st) {
-    if (!wave2d_covers(ndim, p, dd)) return -2;
-    return wave2d_flux<double>(flux, p, S, ph, dd, U, (double*)nullptr, K, cb, st);
+    if (!wave_covers(ndim, p, flux, dd)) return -2;
+    return wave_residual<double>(flux, p, S, ph, dd, U, (double*)nullptr, K, cb, st);
 }
 
 int residual_stage(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                    const float* U, float* K, const StageComb<float>& cb, hipStream_t st) {
-    if (!wave2d_covers(ndim, p, dd)) return -2;
-    return wave2d_flux<float>(flux, p, S, phys_cast<float>(ph), dd, U, (double*)nullptr, K, cb, st);
+    if (!wave_covers(ndim, p, flux, dd)) return -2;
+    return wave_residual<float>(flux, p, S, phys_cast<float>(ph), dd, U, (double*)nullptr, K, cb, st);
 }
 
 template <class PH, int D, class UT = double>
 int dispatch_order(int p, const DevSpace& S, const typename PH::Params& ph, const DiscDev& dd, const UT* U,
                    double* R, hipStream_t st, hipEvent_t* ev) {
+    // P1-P3 in 2D come here with the DDGIC lifting vectors only, 3D fluxes
+    // without a gradient not with P2 and P3 (wave_covers)
+    constexpr bool EULER3 = D == 3 && !TraceRec<PH, D>::NEED_GRAD;
     if (p == 4) return launch_residual<D, 4, PH, UT>(S, ph, dd, U, R, st, ev);
-    // 2D P1-P3 come here with the DDGIC lifting vectors only (wave2d_covers)
     if constexpr (D != 2 || PH::HAS_HOMOGENEITY) {
-        switch (p) {
-        case 1: return launch_residual<D, 1, PH, UT>(S, ph, dd, U, R, st, ev);
-        case 2: return launch_residual<D, 2, PH, UT>(S, ph, dd, U, R, st, ev);
-        case 3: return launch_residual<D, 3, PH, UT>(S, ph, dd, U, R, st, ev);
+        if (p == 1) return launch_residual<D, 1, PH, UT>(S, ph, dd, U, R, st, ev);
+        if constexpr (!EULER3) {
+            if (p == 2) return launch_residual<D, 2, PH, UT>(S, ph, dd, U, R, st, ev);
+            if (p == 3) return launch_residual<D, 3, PH, UT>(S, ph, dd, U, R, st, ev);
         }
     }
     return -1;
@@ -2628,9 +2209,9 @@ int dispatch_order(int p, const DevSpace& S, const typename PH::Params& ph, cons
 
 int residual_fp64(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                   const double* U, double* R, hipStream_t st, hipEvent_t* ev) {
-    if (wave2d_covers(ndim, p, dd))
+    if (wave_covers(ndim, p, flux, dd))
         return profiled(ev, st, [&] {
-            return wave2d_flux<double>(flux, p, S, ph, dd, U, R, (double*)nullptr, StageComb<double>{}, st);
+            return wave_residual<double>(flux, p, S, ph, dd, U, R, (double*)nullptr, StageComb<double>{}, st);
         });
     if (flux == ICE_FLUX_BURGERS) {
         if (ndim == 1) return dispatch_order<Burgers<1>, 1>(p, S, ph, dd, U, R, st, ev);
@@ -2663,8 +2244,8 @@ int residual_mixed_dim(int p, int flux, const DevSpace& S, const PhysParams& ph,
 
 int residual_mixed(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                    const double* U, double* R, hipStream_t st, hipEvent_t* ev) {
-    if (wave2d_covers(ndim, p, dd))
-        return profiled(ev, st, [&] { return wave2d_flux<float>(flux, p, S, phys_cast<float>(ph), dd, U, R, st); });
+    if (wave_covers(ndim, p, flux, dd))
+        return profiled(ev, st, [&] { return wave_residual<float>(flux, p, S, phys_cast<float>(ph), dd, U, R, st); });
     if (ndim == 2) return residual_mixed_dim<2, double>(p, flux, S, ph, dd, U, R, st, ev);
     if (ndim == 3) return residual_mixed_dim<3, double>(p, flux, S, ph, dd, U, R, st, ev);
     return -2;
@@ -2674,8 +2255,8 @@ int residual_mixed(int ndim, int p, int flux, const DevSpace& S, const PhysParam
 // coefficients; differences and element values still formed in FP64)
 int residual_mixed_f32state(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                             const float* U, double* R, hipStream_t st) {
-    if (wave2d_covers(ndim, p, dd))
-        return wave2d_flux<float>(flux, p, S, phys_cast<float>(ph), dd, U, R, (float*)nullptr, StageComb<float>{}, st);
+    if (wave_covers(ndim, p, flux, dd))
+        return wave_residual<float>(flux, p, S, phys_cast<float>(ph), dd, U, R, (float*)nullptr, StageComb<float>{}, st);
     if (ndim == 2) return residual_mixed_dim<2, float>(p, flux, S, ph, dd, U, R, st, nullptr);
     if (ndim == 3) return residual_mixed_dim<3, float>(p, flux, S, ph, dd, U, R, st, nullptr);
     return -2;

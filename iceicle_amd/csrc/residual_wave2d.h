@@ -2,16 +2,8 @@
 // and every contraction is a v_mfma_f64_4x4x4 (four independent 4 x 4 x 4
 // products, one per element).
 //
-// A lane is lo + 4 el + 16 hi.  With N <= 4 nodes per axis an element's
-// N x N tensor, its N x N volume points and its 4 x N face points each fit
-// its 16 (hi, lo) lanes, one value a lane.  The instruction takes A[i][k] at
-// (hi = k, lo = i) and B[k][j] at (hi = k, lo = j) and returns D[i][j] at
-// (hi = i, lo = j), so both operands are contracted over hi, and
-//   data as A, operator as B:  D(hi = the data's lo, lo = new index)
-//   operator as A, data as B:  D(hi = new index, lo = the data's lo).
-// Alternating the two forms contracts one axis after the other with the
-// result of each product already in place for the next: no shuffles, no LDS
-// and no barriers.  Indices beyond N carry zero operators.
+// The element's N x N tensor, its N x N volume points and its 4 x N face
+// points each fit its 16 (hi, lo) lanes (wave_tensor.h), one value a lane.
 //
 // Per wave: the volume term (interpolation, flux, test contraction), the
 // traces of the own faces and of the four neighbours' facing sides
@@ -34,19 +26,9 @@
 #include "kernels.h"
 #include "physics_dev.h"
 #include "stage.h"
+#include "wave_tensor.h"
 
 namespace ice {
-
-__device__ __forceinline__ double mm4(double a, double b, double c) {
-    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
-}
-
-// Consecutive workgroups go to the 8 XCDs in turn; this gives each XCD a
-// contiguous range of workgroups, whose neighbours' coefficients its L2 holds.
-__device__ __forceinline__ int xcd_contiguous(int b, int nblk) {
-    const int q = nblk >> 3, r = nblk & 7, x = b & 7, k = b >> 3;
-    return x * q + (x < r ? x : r) + k;
-}
 
 // Bilinear map x = m + a xi0 + c xi1 + b xi0 xi1 of one element
 struct Quad2 {
@@ -113,19 +95,6 @@ struct FaceSide2 {
         }
     }
 };
-
-// Flux parameters of element e; only Burgers takes a per-element viscosity,
-// the other families read the kernel argument in place.
-template <class PH>
-__device__ __forceinline__ decltype(auto) element_params(const typename PH::Params& p, const double* emu, int e) {
-    if constexpr (PH::HAS_HOMOGENEITY) {
-        typename PH::Params q = p;
-        if (emu) q.mu = (typename PH::real)emu[e];
-        return q;
-    } else {
-        return (p);
-    }
-}
 
 // Waves per SIMD the registers must allow: 3 costs NS some scratch (96 B) and
 // measured 21.2 us against 21.2 at 2 (mixed 19.2 against 20.4); 4 spills
@@ -352,16 +321,7 @@ __global__ __launch_bounds__(256, ICE_WAVE2D_MINW) void wave2d_kernel(DevSpace S
 #pragma unroll
         for (int v = 0; v < M; ++v) r[v] -= dd.srcload[o + v];
     }
-    if (dd.wave) {  // maxima of the wave's points, folded by wave_reduce_kernel
-        for (int off = 32; off > 0; off >>= 1) {
-            lam_w = fmax(lam_w, __shfl_xor(lam_w, off));
-            vis_w = fmax(vis_w, __shfl_xor(vis_w, off));
-        }
-        if (lane == 0) {
-            dd.wave_part[2 * (size_t)wv] = lam_w;
-            dd.wave_part[2 * (size_t)wv + 1] = vis_w;
-        }
-    }
+    if (dd.wave) store_wave_maxima(lam_w, vis_w, wv, dd.wave_part);
     if constexpr (!STAGE) {
         if (store) {
 #pragma unroll
@@ -382,7 +342,10 @@ __global__ __launch_bounds__(256, ICE_WAVE2D_MINW) void wave2d_kernel(DevSpace S
             const double k = mm4(bn, mm4(y, bn, 0.0), 0.0);
             kn[v] = sing ? (UT)(1e-8 * r[v]) : (UT)k;
         }
-        if (store) stage_combine_line<M, UT>(cb, K, o, stage_dt(cb, e), kn);
+        if (store) {
+            if constexpr (std::is_same<UT, double>::value) stage_advance_line<M>(cb, o, stage_dt(cb, e), u0, kn);
+            else stage_combine_line<M, UT>(cb, K, o, stage_dt(cb, e), kn);
+        }
     }
 }
 
