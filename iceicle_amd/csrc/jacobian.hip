@@ -1,4 +1,5 @@
-// Finite-difference element-block Jacobian on the device
+// Finite-difference element-block Jacobian on the device in 3D and with
+// DDGIC vectors (jacobian_rows.hip: 1D and 2D without)
 // (form_petsc_jacobian_fd DG part, form_petsc_jacobian.hpp:55-317, and
 // ConservationLawDDG::domain_integral_jacobian, conservation_law.hpp:316-432).
 //
@@ -766,22 +767,24 @@ int jac_order3(int p, const DevSpace& S, const PhysParams& ph, const DiscDev& dd
     }
 }
 
+// block rows in one launch (jacobian_rows.hip): 1D and 2D without DDGIC vectors
+int jacobian_rows(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
+                  const double* U, double* J, hipStream_t st);
+
 int jacobian_fp64(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                   const double* U, double* J, size_t nvals, hipStream_t st) {
     (void)nvals;
+    // ph's factors and not the vectors' buffer decide: an update may set them to zero
+    const bool ddgic = flux == ICE_FLUX_BURGERS && (ph.sigma_face != 0.0 || ph.sigma_bdy != 0.0);
+    if (ndim < 3 && !ddgic) return jacobian_rows(ndim, p, flux, S, ph, dd, U, J, st);
     if (flux == ICE_FLUX_BURGERS) {
         if (ndim == 1) return jac_order<Burgers<1>, 1>(p, S, ph, dd, U, J, st);
         if (ndim == 2) return jac_order<Burgers<2>, 2>(p, S, ph, dd, U, J, st);
         if (ndim == 3) return jac_order3<Burgers<3>>(p, S, ph, dd, U, J, st);
-    } else if (flux == ICE_FLUX_NAVIER_STOKES) {
-        if (ndim == 1) return jac_order<NavierStokes<1, true>, 1>(p, S, ph, dd, U, J, st);
-        if (ndim == 2) return jac_order<NavierStokes<2, true>, 2>(p, S, ph, dd, U, J, st);
-        if (ndim == 3) return jac_order3<NavierStokes<3, true>>(p, S, ph, dd, U, J, st);
-    } else if (flux == ICE_FLUX_EULER) {
-        if (ndim == 1) return jac_order<NavierStokes<1, false>, 1>(p, S, ph, dd, U, J, st);
-        if (ndim == 2) return jac_order<NavierStokes<2, false>, 2>(p, S, ph, dd, U, J, st);
-        if (ndim == 3) return jac_order3<NavierStokes<3, false>>(p, S, ph, dd, U, J, st);
     }
+    if (ndim != 3) return -1;
+    if (flux == ICE_FLUX_NAVIER_STOKES) return jac_order3<NavierStokes<3, true>>(p, S, ph, dd, U, J, st);
+    if (flux == ICE_FLUX_EULER) return jac_order3<NavierStokes<3, false>>(p, S, ph, dd, U, J, st);
     return -1;
 }
 
