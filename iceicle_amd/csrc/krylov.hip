@@ -658,34 +658,39 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
     return s;
 }
 
-// partial[blk][j] = sum_i V_j[i] w[i] for j < nv, partial[blk][nv] = w.w
+// partial[blk][j] = sum_i V_j[i] w[i] for j < nv, partial[blk][nv] = w.w; a
+// workgroup takes MDOT_VECS of the vectors over one chunk of w, so that a
+// vector of few chunks still fills the chip (128 chunks of 262k entries, 15
+// vectors one after another: 51 us; 2D grid: 17 us)
+constexpr int MDOT_VECS = 4;
 __global__ __launch_bounds__(256) void mdot_partial_kernel(size_t n, int nv, const double* __restrict__ V, size_t ldv,
                                                            const double* __restrict__ w, double* __restrict__ part,
                                                            int npart) {
-    __shared__ double red[4];
+    __shared__ double red[4][MDOT_VECS];
     const size_t base = (size_t)blockIdx.x * blockDim.x * VEC_EPT + threadIdx.x;
-    double wr[VEC_EPT];
+    const int j0 = blockIdx.y * MDOT_VECS;
+    // vector nv is w itself; beyond it w again, dropped
+    const double* vp[MDOT_VECS];
+#pragma unroll
+    for (int k = 0; k < MDOT_VECS; ++k) vp[k] = j0 + k < nv ? V + (size_t)(j0 + k) * ldv : w;
+    double s[MDOT_VECS] = {};
 #pragma unroll
     for (int e = 0; e < VEC_EPT; ++e) {
-        const size_t i = base + (size_t)e * blockDim.x;
-        wr[e] = (i < n) ? w[i] : 0.0;
-    }
-    for (int j = 0; j <= nv; ++j) {
-        double s = 0.0;
-        if (j < nv) {
-            const double* vj = V + (size_t)j * ldv;
+        const size_t i = base + (size_t)e * blockDim.x, ic = i < n ? i : n - 1;
+        const double wi = w[ic];
 #pragma unroll
-            for (int e = 0; e < VEC_EPT; ++e) {
-                const size_t i = base + (size_t)e * blockDim.x;
-                if (i < n) s += vj[i] * wr[e];
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < VEC_EPT; ++e) s += wr[e] * wr[e];
-        }
-        s = block_sum(s, red);
-        if (threadIdx.x == 0) part[(size_t)blockIdx.x * npart + j] = s;
+        for (int k = 0; k < MDOT_VECS; ++k) s[k] += i < n ? vp[k][ic] * wi : 0.0;
     }
+#pragma unroll
+    for (int k = 0; k < MDOT_VECS; ++k)
+        for (int off = 32; off > 0; off >>= 1) s[k] += __shfl_xor(s[k], off);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int k = 0; k < MDOT_VECS; ++k) red[threadIdx.x >> 6][k] = s[k];
+    __syncthreads();
+    if (threadIdx.x < MDOT_VECS && j0 + (int)threadIdx.x <= nv)
+        part[(size_t)blockIdx.x * npart + j0 + threadIdx.x] =
+            (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
 // out[j] = sum_blk part[blk][j], one workgroup per j
@@ -699,30 +704,34 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(int nblk, const do
     if (threadIdx.x == 0) out[j] = s;
 }
 
-// w -= sum_j h[j] V_j ; partial[blk] = w.w afterwards
+// w -= sum_j h[j] V_j ; partial[blk] = w.w afterwards (MAXPY_EPT entries a
+// thread: four times the workgroups of the reduction's chunks, 29 -> 11 us at
+// 262k entries)
+constexpr int MAXPY_EPT = 2;
 __global__ __launch_bounds__(256) void maxpy_norm_kernel(size_t n, int nv, const double* __restrict__ V, size_t ldv,
                                                          const double* __restrict__ h, double* __restrict__ w,
                                                          double* __restrict__ part) {
     __shared__ double red[4];
-    const size_t base = (size_t)blockIdx.x * blockDim.x * VEC_EPT + threadIdx.x;
-    double acc[VEC_EPT];
+    const size_t base = (size_t)blockIdx.x * blockDim.x * MAXPY_EPT + threadIdx.x;
+    double acc[MAXPY_EPT];
 #pragma unroll
-    for (int e = 0; e < VEC_EPT; ++e) {
+    for (int e = 0; e < MAXPY_EPT; ++e) {
         const size_t i = base + (size_t)e * blockDim.x;
         acc[e] = (i < n) ? w[i] : 0.0;
     }
+#pragma unroll 4
     for (int j = 0; j < nv; ++j) {
         const double hj = h[j];
         const double* vj = V + (size_t)j * ldv;
 #pragma unroll
-        for (int e = 0; e < VEC_EPT; ++e) {
+        for (int e = 0; e < MAXPY_EPT; ++e) {
             const size_t i = base + (size_t)e * blockDim.x;
             if (i < n) acc[e] -= hj * vj[i];
         }
     }
     double s = 0.0;
 #pragma unroll
-    for (int e = 0; e < VEC_EPT; ++e) {
+    for (int e = 0; e < MAXPY_EPT; ++e) {
         const size_t i = base + (size_t)e * blockDim.x;
         if (i < n) {
             w[i] = acc[e];
@@ -758,37 +767,54 @@ __global__ void axpby_kernel2(size_t n, double a, const double* __restrict__ x, 
         y[i] = (a == 0.0 ? 0.0 : a * x[i]) + (b == 0.0 ? 0.0 : b * y[i]);
 }
 
-// Arnoldi bookkeeping of step k (one thread): column k of the Hessenberg
-// matrix from the two Gram-Schmidt passes, the norm of the new vector,
-// Givens rotations, residual estimate.  sc layout: see GmresScalars.
-__global__ void arnoldi_kernel(int k, int m, const double* __restrict__ h1, const double* __restrict__ h2,
-                               int refine, double* __restrict__ sc) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// Arnoldi bookkeeping of step k (one workgroup): the norm of the new vector
+// from its nblk partial sums, column k of the Hessenberg matrix from the
+// Gram-Schmidt passes, Givens rotations, residual estimate.  sc layout: see
+// GmresScalars.  The rotations are a serial chain, taken by one thread from
+// LDS.
+__global__ __launch_bounds__(256) void arnoldi_kernel(int k, int m, const double* __restrict__ h1,
+                                                      const double* __restrict__ h2, int refine,
+                                                      const double* __restrict__ part, int nblk,
+                                                      double* __restrict__ sc) {
+    extern __shared__ double sh[];  // column [m + 1], cs [m], sn [m]
+    __shared__ double red[4];
     double* H = sc;                       // (m+1) x m, column-major: H[j + (m+1) k]
     double* cs = H + (size_t)(m + 1) * m;
     double* sn = cs + m;
     double* g = sn + m;                   // m+1
     double* hn = g + m + 1;               // [0] = ||v_{k+1}|| before normalisation, [1] = |g_{k+1}|
     double* col = H + (size_t)(m + 1) * k;
-    for (int j = 0; j <= k; ++j) col[j] = refine ? h1[j] + h2[j] : h1[j];
-    const double hk1 = sqrt(fmax(h2[k + 1], 0.0));  // h2[k+1] = squared norm after the last pass
-    col[k + 1] = hk1;
-    hn[0] = hk1;
-    for (int j = 0; j < k; ++j) {
-        const double a = col[j], b = col[j + 1];
-        col[j] = cs[j] * a + sn[j] * b;
-        col[j + 1] = -sn[j] * a + cs[j] * b;
+    double *scol = sh, *scs = sh + m + 1, *ssn = scs + m;
+    double nrm2 = 0.0;
+    for (int b = threadIdx.x; b < nblk; b += blockDim.x) nrm2 += part[b];
+    for (int j = threadIdx.x; j <= k; j += blockDim.x) {
+        scol[j] = refine ? h1[j] + h2[j] : h1[j];
+        scs[j] = cs[j];
+        ssn[j] = sn[j];
     }
-    const double a = col[k], b = col[k + 1];
-    const double r = hypot(a, b);
-    const double c = (r > 0.0) ? a / r : 1.0, s = (r > 0.0) ? b / r : 0.0;
-    cs[k] = c;
-    sn[k] = s;
-    col[k] = r;
-    col[k + 1] = 0.0;
-    g[k + 1] = -s * g[k];
-    g[k] = c * g[k];
-    hn[1] = fabs(g[k + 1]);
+    nrm2 = block_sum(nrm2, red);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const double hk1 = sqrt(fmax(nrm2, 0.0));
+        hn[0] = hk1;
+        double a = scol[0];
+        for (int j = 0; j < k; ++j) {
+            const double b = scol[j + 1];
+            scol[j] = scs[j] * a + ssn[j] * b;
+            a = -ssn[j] * a + scs[j] * b;
+        }
+        const double r = hypot(a, hk1);
+        const double c = (r > 0.0) ? a / r : 1.0, s = (r > 0.0) ? hk1 / r : 0.0;
+        cs[k] = c;
+        sn[k] = s;
+        scol[k] = r;
+        col[k + 1] = 0.0;
+        g[k + 1] = -s * g[k];
+        g[k] = c * g[k];
+        hn[1] = fabs(g[k + 1]);
+    }
+    __syncthreads();
+    for (int j = threadIdx.x; j <= k; j += blockDim.x) col[j] = scol[j];
 }
 
 // back substitution H(0:k,0:k) y = g(0:k), result into y
@@ -819,21 +845,21 @@ int vec_grid(size_t n) { return (int)((n + 256 * VEC_EPT - 1) / (256 * VEC_EPT))
 
 }  // namespace
 
-int gmres_partials(size_t n) { return vec_grid(n); }
+int maxpy_grid(size_t n) { return (int)((n + 256 * MAXPY_EPT - 1) / (256 * MAXPY_EPT)); }
+
+int gmres_partials(size_t n) { return maxpy_grid(n); }
 
 int launch_mdot(size_t n, int nv, const double* V, size_t ldv, const double* w, double* part, int npart, double* out,
                 hipStream_t st) {
     const int nb = vec_grid(n);
-    mdot_partial_kernel<<<nb, 256, 0, st>>>(n, nv, V, ldv, w, part, npart);
+    mdot_partial_kernel<<<dim3(nb, nv / MDOT_VECS + 1), 256, 0, st>>>(n, nv, V, ldv, w, part, npart);
     reduce_partials_kernel<<<nv + 1, 256, 0, st>>>(nb, part, npart, out);
     return (int)hipGetLastError();
 }
 
 int launch_maxpy_norm(size_t n, int nv, const double* V, size_t ldv, const double* h, double* w, double* part,
-                      double* out, hipStream_t st) {
-    const int nb = vec_grid(n);
-    maxpy_norm_kernel<<<nb, 256, 0, st>>>(n, nv, V, ldv, h, w, part);
-    if (out) reduce_partials_kernel<<<1, 256, 0, st>>>(nb, part, 1, out);
+                      hipStream_t st) {
+    maxpy_norm_kernel<<<maxpy_grid(n), 256, 0, st>>>(n, nv, V, ldv, h, w, part);
     return (int)hipGetLastError();
 }
 
@@ -856,8 +882,9 @@ int launch_axpby2(size_t n, double a, const double* x, double b, double* y, hipS
     return (int)hipGetLastError();
 }
 
-int launch_arnoldi(int k, int m, const double* h1, const double* h2, int refine, double* sc, hipStream_t st) {
-    arnoldi_kernel<<<1, 64, 0, st>>>(k, m, h1, h2, refine, sc);
+int launch_arnoldi(size_t n, int k, int m, const double* h1, const double* h2, int refine, const double* part,
+                   double* sc, hipStream_t st) {
+    arnoldi_kernel<<<1, 256, (size_t)(3 * m + 1) * sizeof(double), st>>>(k, m, h1, h2, refine, part, maxpy_grid(n), sc);
     return (int)hipGetLastError();
 }
 
@@ -1395,65 +1422,53 @@ int convert_transpose_fp32(size_t nblocks, int bs, const double* a, float* b, hi
 
 // FP32 (and optionally FP16) column-major copies of row-major FP64 blocks,
 // one workgroup per block: the block is read once, coalesced, into LDS and
-// both copies are written coalesced from it.
-__global__ __launch_bounds__(256) void convert_transpose_tile_kernel(int bs, const double* __restrict__ a,
+// both copies are written coalesced from it.  With ap, the block's columns
+// summed over the basis, ap[w][r] = sum_j a[r][j m + w] (the block applied to
+// element constants, for the multigrid), and their sums over the row nodes,
+// a0[v][w] = sum_i ap[w][i m + v] (the level-0 Galerkin block), from the same
+// read.
+__global__ __launch_bounds__(256) void convert_transpose_tile_kernel(int bs, int m, const double* __restrict__ a,
                                                                       float* __restrict__ b32,
-                                                                      _Float16* __restrict__ b16) {
+                                                                      _Float16* __restrict__ b16,
+                                                                      float* __restrict__ ap,
+                                                                      double* __restrict__ a0) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int ld = bs | 1;  // odd row stride: the column reads fall on distinct banks
     double* t = reinterpret_cast<double*>(smem_raw);
+    double* q = t + (size_t)bs * ld;  // [w][r]
     const size_t bb = (size_t)bs * bs;
     const double* src = a + (size_t)blockIdx.x * bb;
-    for (int k = threadIdx.x; k < (int)bb; k += blockDim.x) t[k] = src[k];
+    for (int k = threadIdx.x; k < (int)bb; k += blockDim.x) t[(k / bs) * ld + k % bs] = src[k];
     __syncthreads();
     float* d32 = b32 + (size_t)blockIdx.x * bb;
     for (int k = threadIdx.x; k < (int)bb; k += blockDim.x) {
         const int c = k / bs, r = k - c * bs;  // destination [c][r]
-        const float v = (float)t[r * bs + c];
+        const float v = (float)t[r * ld + c];
         d32[k] = v;
         if (b16) b16[(size_t)blockIdx.x * bb + k] = (_Float16)v;
     }
-}
-
-// x = A^-1 b with the dense inverse stored column-major (the multigrid's
-// coarsest level): a workgroup owns 64 rows, its 16 waves split the columns
-// (coalesced column reads, one lane per row), and the 16 partial sums of a
-// row are added in a fixed order from LDS
-__global__ __launch_bounds__(1024) void dense_inverse_apply_kernel(int n, const double* __restrict__ inv,
-                                                                   const double* __restrict__ b,
-                                                                   double* __restrict__ x) {
-    __shared__ double part[16][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int i = blockIdx.x * 64 + lane;
-    const int len = (n + 15) / 16;
-    const int j0 = w * len, j1 = min(n, j0 + len);
-    double s0 = 0.0, s1 = 0.0;
-    if (i < n) {
-        int j = j0;
-        for (; j + 1 < j1; j += 2) {
-            s0 += inv[(size_t)j * n + i] * b[j];
-            s1 += inv[(size_t)(j + 1) * n + i] * b[j + 1];
-        }
-        if (j < j1) s0 += inv[(size_t)j * n + i] * b[j];
+    if (!ap) return;
+    for (int k = threadIdx.x; k < bs * m; k += blockDim.x) {
+        const int w = k / bs, r = k - w * bs;
+        double s = 0.0;
+        for (int c = w; c < bs; c += m) s += t[r * ld + c];
+        q[k] = s;
+        ap[(size_t)blockIdx.x * bs * m + k] = (float)s;
     }
-    part[w][lane] = s0 + s1;
     __syncthreads();
-    if (w == 0 && i < n) {
-        double sacc = 0.0;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) sacc += part[k][lane];
-        x[i] = sacc;
+    for (int k = threadIdx.x; k < m * m; k += blockDim.x) {
+        const int v = k / m, w = k - v * m;
+        double s = 0.0;
+        for (int r = v; r < bs; r += m) s += q[w * bs + r];
+        a0[(size_t)blockIdx.x * m * m + k] = s;
     }
 }
 
-int dense_inverse_apply(int n, const double* inv, const double* b, double* x, hipStream_t st) {
-    dense_inverse_apply_kernel<<<(n + 63) / 64, 1024, 0, st>>>(n, inv, b, x);
-    return (int)hipGetLastError();
-}
-
-int convert_transpose_blocks(size_t nblocks, int bs, const double* a, float* b32, _Float16* b16, hipStream_t st) {
-    const size_t sh = (size_t)bs * bs * sizeof(double);
+int convert_transpose_blocks(size_t nblocks, int bs, int m, const double* a, float* b32, _Float16* b16, float* ap,
+                             double* a0, hipStream_t st) {
+    const size_t sh = ((size_t)bs * (bs | 1) + (ap ? (size_t)bs * m : 0)) * sizeof(double);
     if (sh > 160 * 1024 || nblocks == 0) return nblocks == 0 ? 0 : -1;
-    convert_transpose_tile_kernel<<<(unsigned)nblocks, 256, sh, st>>>(bs, a, b32, b16);
+    convert_transpose_tile_kernel<<<(unsigned)nblocks, 256, sh, st>>>(bs, m, a, b32, b16, ap, a0);
     return (int)hipGetLastError();
 }
 
@@ -1469,25 +1484,6 @@ int convert_transpose_blocks(size_t nblocks, int bs, const double* a, float* b32
 
 namespace ice {
 namespace {
-
-// A0[e][s][v][w] = sum_{i,j} J[e][s][i m + v][j m + w]  (R J P with P the
-// injection of element constants, R = P^T); row-major FP64
-__global__ void galerkin_p0_kernel(int nelem, int nslots, int nb, int m, const double* __restrict__ J,
-                                   double* __restrict__ A0) {
-    const long tid = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    const long total = (long)nelem * nslots * m * m;
-    if (tid >= total) return;
-    const int w = (int)(tid % m), v = (int)((tid / m) % m);
-    const long es = tid / (m * m);
-    const int bs = nb * m;
-    const double* B = J + es * (long)bs * bs;
-    double acc = 0.0;
-    for (int i = 0; i < nb; ++i) {
-        const double* row = B + (long)(i * m + v) * bs + w;
-        for (int j = 0; j < nb; ++j) acc += row[j * m];
-    }
-    A0[tid] = acc;
-}
 
 // Ac[C][s][v][w] = sum over children c of C and slots t of c whose column
 // cell maps to slot s of C (the diagonal when it is a sibling)
@@ -1525,48 +1521,10 @@ __global__ void restrict_nodes_kernel(int nelem, int nb, int m, const double* __
     b0[tid] = acc;
 }
 
-// x[e][i][v] += x0[e][v]
-__global__ void prolong_nodes_kernel(int nelem, int nb, int m, const double* __restrict__ x0, double* __restrict__ x) {
-    const long tid = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    const long total = (long)nelem * nb * m;
-    if (tid >= total) return;
-    const int v = (int)(tid % m);
-    const long e = tid / ((long)nb * m);
-    x[tid] += x0[e * m + v];
-}
-
-// bc[C][v] = sum over children of r[c][v]
-__global__ void restrict_agg_kernel(int ncoarse, int m, const int* __restrict__ children, const double* __restrict__ r,
-                                    double* __restrict__ bc) {
-    const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (tid >= ncoarse * m) return;
-    const int C = tid / m, v = tid - C * m;
-    double acc = 0.0;
-    for (int k = 0; k < 8; ++k) {
-        const int c = children[C * 8 + k];
-        if (c >= 0) acc += r[(size_t)c * m + v];
-    }
-    bc[tid] = acc;
-}
-
-// x[c][v] += xc[parent(c)][v]
-__global__ void prolong_agg_kernel(int nfine, int m, const int* __restrict__ parent, const double* __restrict__ xc,
-                                   double* __restrict__ x) {
-    const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (tid >= nfine * m) return;
-    const int c = tid / m, v = tid - c * m;
-    x[tid] += xc[(size_t)parent[c] * m + v];
-}
-
 inline int grid_of(long n) { return (int)((n + 255) / 256); }
 
 }  // namespace
 
-int mg_galerkin_p0(int nelem, int nslots, int nb, int m, const double* J, double* A0, hipStream_t st) {
-    const long total = (long)nelem * nslots * m * m;
-    galerkin_p0_kernel<<<grid_of(total), 256, 0, st>>>(nelem, nslots, nb, m, J, A0);
-    return (int)hipGetLastError();
-}
 int mg_galerkin_agg(int ncoarse, int nslots, int m, const int* children, const int* fcols, const int* parent,
                     const double* Af, double* Ac, hipStream_t st) {
     const long total = (long)ncoarse * nslots * m * m;
@@ -1575,18 +1533,6 @@ int mg_galerkin_agg(int ncoarse, int nslots, int m, const int* children, const i
 }
 int mg_restrict_nodes(int nelem, int nb, int m, const double* r, double* b0, hipStream_t st) {
     restrict_nodes_kernel<<<grid_of((long)nelem * m), 256, 0, st>>>(nelem, nb, m, r, b0);
-    return (int)hipGetLastError();
-}
-int mg_prolong_nodes(int nelem, int nb, int m, const double* x0, double* x, hipStream_t st) {
-    prolong_nodes_kernel<<<grid_of((long)nelem * nb * m), 256, 0, st>>>(nelem, nb, m, x0, x);
-    return (int)hipGetLastError();
-}
-int mg_restrict_agg(int ncoarse, int m, const int* children, const double* r, double* bc, hipStream_t st) {
-    restrict_agg_kernel<<<grid_of((long)ncoarse * m), 256, 0, st>>>(ncoarse, m, children, r, bc);
-    return (int)hipGetLastError();
-}
-int mg_prolong_agg(int nfine, int m, const int* parent, const double* xc, double* x, hipStream_t st) {
-    prolong_agg_kernel<<<grid_of((long)nfine * m), 256, 0, st>>>(nfine, m, parent, xc, x);
     return (int)hipGetLastError();
 }
 

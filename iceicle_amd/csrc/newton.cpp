@@ -21,6 +21,7 @@
 #include "engine.h"
 #include "kernels.h"
 #include "linesearch.h"
+#include "mg.h"
 
 namespace ice {
 // krylov.hip
@@ -36,19 +37,15 @@ template <class T, class V, class TD>
 int sgsT_sweep(bool forward, int nel, const int* elems, const int* ecolor, int colour, int nslots, int bs,
                const int* cols, const T* JT, const TD* DT, const V* rhs, V* y, hipStream_t st);
 int convert_transpose_fp32(size_t nblocks, int bs, const double* a, float* b, hipStream_t st);
-int convert_transpose_blocks(size_t nblocks, int bs, const double* a, float* b32, _Float16* b16, hipStream_t st);
-int dense_inverse_apply(int n, const double* inv, const double* b, double* x, hipStream_t st);
+int convert_transpose_blocks(size_t nblocks, int bs, int m, const double* a, float* b32, _Float16* b16, float* ap,
+                             double* a0, hipStream_t st);
 int line_factor(int nelem, int nslots, int bs, const double* J, double* Sinv, double* W, int* nsingular,
                 hipStream_t st);
 int line_solve(int nelem, int nslots, int bs, const double* J, const double* Sinv, const double* W, const double* b,
                double* x, hipStream_t st);
-int mg_galerkin_p0(int nelem, int nslots, int nb, int m, const double* J, double* A0, hipStream_t st);
 int mg_galerkin_agg(int ncoarse, int nslots, int m, const int* children, const int* fcols, const int* parent,
                     const double* Af, double* Ac, hipStream_t st);
 int mg_restrict_nodes(int nelem, int nb, int m, const double* r, double* b0, hipStream_t st);
-int mg_prolong_nodes(int nelem, int nb, int m, const double* x0, double* x, hipStream_t st);
-int mg_restrict_agg(int ncoarse, int m, const int* children, const double* r, double* bc, hipStream_t st);
-int mg_prolong_agg(int nfine, int m, const int* parent, const double* xc, double* x, hipStream_t st);
 template <class T, class V>
 int block_diag_apply(int nelem, int bs, const T* D, const V* x, V* y, hipStream_t st);
 int convert_to_fp32(size_t n, const double* a, float* b, hipStream_t st);
@@ -56,12 +53,13 @@ int gmres_partials(size_t n);
 int launch_mdot(size_t n, int nv, const double* V, size_t ldv, const double* w, double* part, int npart, double* out,
                 hipStream_t st);
 int launch_maxpy_norm(size_t n, int nv, const double* V, size_t ldv, const double* h, double* w, double* part,
-                      double* out, hipStream_t st);
+                      hipStream_t st);
 int launch_norm2(size_t n, const double* w, double* part, double* out, hipStream_t st);
 int launch_combine(size_t n, int nv, const double* V, size_t ldv, const double* y, double* x, hipStream_t st);
 int launch_scale(size_t n, const double* s, int inv, double* x, hipStream_t st);
 int launch_axpby2(size_t n, double a, const double* x, double b, double* y, hipStream_t st);
-int launch_arnoldi(int k, int m, const double* h1, const double* h2, int refine, double* sc, hipStream_t st);
+int launch_arnoldi(size_t n, int k, int m, const double* h1, const double* h2, int refine, const double* part,
+                   double* sc, hipStream_t st);
 int launch_hessenberg_solve(int k, int m, const double* sc, double* y, hipStream_t st);
 int launch_gmres_init(int m, const double* nrm2, double* sc, hipStream_t st);
 template <class T, class V>
@@ -99,13 +97,14 @@ struct MGLevel {
     int n = 0;
     int dims[3] = {1, 1, 1};
     std::vector<int> hcols;        // [n][nslots]
+    std::vector<int> at;           // [n] lexicographic grid position (level 0: the cell number)
     const int* cols = nullptr;     // device copy of hcols
     int* parent = nullptr;         // [n] cell of the next coarser level (null on the coarsest)
     int* children = nullptr;       // [n][8] cells of the next finer level (level 0: none)
     double* A64 = nullptr;         // [n][nslots][m][m] row-major
-    float* A32 = nullptr;          // column-major FP32 copy
-    float* Dinv = nullptr;         // column-major factored diagonal blocks
-    int* ecolor = nullptr;
+    float* A32 = nullptr;          // FP32 copy and factored diagonal blocks (MGCells)
+    float* Dinv = nullptr;
+    int* ecolor = nullptr;         // level 0 only: the others are numbered colour by colour
     int* celems = nullptr;
     std::vector<int> coff;
     double *x = nullptr, *b = nullptr, *r = nullptr, *t = nullptr;
@@ -140,9 +139,13 @@ struct ice_newton {
     double* line_W = nullptr;
     std::vector<MGLevel> mg;    // multigrid levels (level 0 = element constants)
     double *mg_r = nullptr, *mg_t = nullptr;  // fine-level work vectors of the V-cycle
+    float* mg_d = nullptr;      // a level's factored diagonals before they are packed
+    bool fine_fused = false;    // the fine residual is restricted by the kernel that forms it
+    float* fine_ap = nullptr;   // [nelem][nslots][neq][bs]: the blocks applied to element constants
     double* coarse_inv = nullptr;  // dense inverse of the coarsest level (column-major), when it is small
     int coarse_n = 0;
-    bool coarse_direct = false;    // this factorisation's coarsest level is solved exactly
+    ice::MGTail tail{};            // levels from tail_level on, taken by one workgroup
+    int tail_level = 0;
     int neq = 0, nbasis = 0;
     int* ecolor = nullptr;      // element colour (multicolour Gauss-Seidel)
     int* celems = nullptr;      // elements grouped by colour
@@ -222,10 +225,11 @@ struct ice_newton {
         else NT_LAUNCH((ice::block_diag_apply<double, double>(nelem, bs, (const double*)Dinv, v, out, st)));
     }
 
-    // greedy colouring of a block graph (face neighbours differ); returns the
-    // colour offsets, fills the device colour and grouped-cell arrays
-    std::vector<int> colour_graph(int ncell, const std::vector<int>& cols, int** dcolour, int** dcells) {
-        std::vector<int> col(ncell, -1);
+    // greedy colouring of a block graph (face neighbours differ): the colour
+    // offsets, each cell's colour and the cells grouped by colour
+    std::vector<int> colour_cells(int ncell, const std::vector<int>& cols, std::vector<int>& col,
+                                  std::vector<int>& order) const {
+        col.assign(ncell, -1);
         int nc = 0;
         for (int e = 0; e < ncell; ++e) {
             unsigned used = 0;
@@ -241,8 +245,14 @@ struct ice_newton {
         std::vector<int> off(nc + 1, 0);
         for (int e = 0; e < ncell; ++e) ++off[col[e] + 1];
         for (int c = 0; c < nc; ++c) off[c + 1] += off[c];
-        std::vector<int> order(ncell), fill(off.begin(), off.end() - 1);
+        order.resize(ncell);
+        std::vector<int> fill(off.begin(), off.end() - 1);
         for (int e = 0; e < ncell; ++e) order[fill[col[e]]++] = e;
+        return off;
+    }
+    std::vector<int> colour_graph(int ncell, const std::vector<int>& cols, int** dcolour, int** dcells) {
+        std::vector<int> col, order;
+        std::vector<int> off = colour_cells(ncell, cols, col, order);
         *dcolour = alloc<int>(ncell);
         *dcells = alloc<int>(ncell);
         NT_HIP(hipMemcpy(*dcolour, col.data(), ncell * sizeof(int), hipMemcpyHostToDevice));
@@ -257,45 +267,46 @@ struct ice_newton {
         coff = colour_graph(nelem, cols, &ecolor, &celems);
     }
 
+    ice::MGCells cells(int l) const {
+        const MGLevel& L = mg[l];
+        ice::MGCells c{};
+        c.n = L.n;
+        c.ncol = (int)L.coff.size() - 1;
+        c.cols = L.cols;
+        c.A = L.A32;
+        c.Dinv = L.Dinv;
+        c.ecolor = L.ecolor;
+        c.celems = L.celems;
+        for (int k = 0; k <= c.ncol; ++k) c.coff[k] = L.coff[k];
+        c.children = L.children;
+        c.parent = L.parent;
+        return c;
+    }
+
     // out = M^-1 rhs for one multicolour block SGS sweep with m x m blocks on level L
-    void sgs_level(const MGLevel& L, const double* rhs, double* out, hipStream_t st) {
-        const int nc = (int)L.coff.size() - 1;
-        for (int pass = 0; pass < 2; ++pass)
-            for (int k = 0; k < nc; ++k) {
-                const bool fwd = pass == 0;
-                const int c = fwd ? k : nc - 1 - k;
-                if (!fwd && c == nc - 1) continue;
-                NT_LAUNCH((ice::sgsT_sweep<float, double, float>(fwd, L.coff[c + 1] - L.coff[c], L.celems + L.coff[c],
-                                                          L.ecolor, c, nslots, neq, L.cols, L.A32, L.Dinv, rhs, out,
-                                                          st)));
-            }
+    void sgs_level(const ice::MGCells& L, const double* rhs, double* out, hipStream_t st) {
+        if (L.ncol == 2) {
+            NT_LAUNCH(ice::mg_forward2(nslots, neq, L, rhs, out, st));
+        } else {
+            for (int c = 0; c < L.ncol; ++c) NT_LAUNCH(ice::mg_forward(nslots, neq, L, c, rhs, out, st));
+        }
+        for (int c = L.ncol - 2; c >= 0; --c) NT_LAUNCH(ice::mg_backward(nslots, neq, L, c, out, st));
     }
 
     // x = V-cycle approximation of A_l^-1 b (x need not be initialised)
     void vcycle(int l, const double* b, double* x, hipStream_t st) {
-        MGLevel& L = mg[l];
-        const size_t nl = (size_t)L.n * neq;
-        if (l + 1 == (int)mg.size() && coarse_direct) {
-            NT_LAUNCH(ice::dense_inverse_apply(coarse_n, coarse_inv, b, x, st));
-            return;
-        }
-        sgs_level(L, b, x, st);
-        if (l + 1 == (int)mg.size()) {
-            for (int it = 0; it < 8; ++it) {
-                NT_LAUNCH((ice::bsrT_apply<float, double>(L.n, nslots, neq, L.cols, L.A32, x, b, L.r, st)));
-                sgs_level(L, L.r, L.t, st);
-                NT_LAUNCH(ice::launch_axpby2(nl, 1.0, L.t, 1.0, x, st));
-            }
+        if (l >= tail_level) {
+            NT_LAUNCH(ice::mg_tail_cycle(nslots, neq, tail, b, x, st));
             return;
         }
         MGLevel& Cn = mg[l + 1];
-        NT_LAUNCH((ice::bsrT_apply<float, double>(L.n, nslots, neq, L.cols, L.A32, x, b, L.r, st)));
-        NT_LAUNCH(ice::mg_restrict_agg(Cn.n, neq, Cn.children, L.r, Cn.b, st));
+        const ice::MGCells L = cells(l), C = cells(l + 1);
+        sgs_level(L, b, x, st);
+        NT_LAUNCH(ice::mg_residual_restrict(nslots, neq, L, C, b, x, Cn.b, st));
         vcycle(l + 1, Cn.b, Cn.x, st);
-        NT_LAUNCH(ice::mg_prolong_agg(L.n, neq, L.parent, Cn.x, x, st));
-        NT_LAUNCH((ice::bsrT_apply<float, double>(L.n, nslots, neq, L.cols, L.A32, x, b, L.r, st)));
-        sgs_level(L, L.r, L.t, st);
-        NT_LAUNCH(ice::launch_axpby2(nl, 1.0, L.t, 1.0, x, st));
+        NT_LAUNCH(ice::mg_prolong_residual(nslots, neq, L, b, x, Cn.x, mg[l].r, st));
+        sgs_level(L, mg[l].r, mg[l].t, st);
+        NT_LAUNCH(ice::mg_prolong_add(neq, L, Cn.x, mg[l].t, x, st));
     }
 
     // hierarchy structure: level 0 = the elements, then 2^ndim agglomerates
@@ -322,7 +333,8 @@ struct ice_newton {
             C.n = C.dims[0] * C.dims[1] * C.dims[2];
             std::vector<int> par(F.n), ch((size_t)C.n * 8, -1), cnt(C.n, 0);
             for (int c = 0; c < F.n; ++c) {
-                const int i = c % F.dims[0], j = (c / F.dims[0]) % F.dims[1], k = c / (F.dims[0] * F.dims[1]);
+                const int at = F.at.empty() ? c : F.at[c];
+                const int i = at % F.dims[0], j = (at / F.dims[0]) % F.dims[1], k = at / (F.dims[0] * F.dims[1]);
                 const int P = i / 2 + C.dims[0] * (j / 2 + C.dims[1] * (k / 2));
                 par[c] = P;
                 ch[(size_t)P * 8 + cnt[P]++] = c;
@@ -335,6 +347,24 @@ struct ice_newton {
                     if (col < 0 || par[col] == par[c]) continue;
                     C.hcols[(size_t)par[c] * nslots + t] = par[col];
                 }
+            // the level's cells renumbered colour by colour
+            std::vector<int> col, order, id(C.n);
+            C.coff = colour_cells(C.n, C.hcols, col, order);
+            for (int k = 0; k < C.n; ++k) id[order[k]] = k;
+            std::vector<int> hc(C.hcols.size()), ch2(ch.size());
+            for (int k = 0; k < C.n; ++k) {
+                for (int t = 0; t < nslots; ++t) {
+                    const int c2 = C.hcols[(size_t)order[k] * nslots + t];
+                    hc[(size_t)k * nslots + t] = c2 < 0 ? -1 : id[c2];
+                }
+                for (int t = 0; t < 8; ++t) ch2[(size_t)k * 8 + t] = ch[(size_t)order[k] * 8 + t];
+            }
+            C.hcols.swap(hc);
+            ch.swap(ch2);
+            for (int& P : par) P = id[P];
+            // grid position of the renumbered cells, for the next level
+            C.at.resize(C.n);
+            for (int k = 0; k < C.n; ++k) C.at[k] = order[k];
             F.parent = alloc<int>(F.n);
             NT_HIP(hipMemcpy(F.parent, par.data(), F.n * sizeof(int), hipMemcpyHostToDevice));
             C.children = alloc<int>((size_t)C.n * 8);
@@ -350,10 +380,27 @@ struct ice_newton {
             L.A32 = alloc<float>(nb2);
             L.Dinv = alloc<float>((size_t)L.n * neq * neq);
             for (double** v : {&L.x, &L.b, &L.r, &L.t}) *v = alloc<double>((size_t)L.n * neq);
-            L.coff = colour_graph(L.n, L.hcols, &L.ecolor, &L.celems);
+            if (L.coff.empty()) L.coff = colour_graph(L.n, L.hcols, &L.ecolor, &L.celems);
         }
+        mg_d = alloc<float>((size_t)nelem * neq * neq);
         mg_r = alloc<double>(n);
         mg_t = alloc<double>(n);
+        if (mg.size() > (size_t)ice::MG_MAX_LEVELS) throw Fail{ICE_ERR_UNSUPPORTED, "too many multigrid levels"};
+        for (const MGLevel& L : mg)
+            if (L.coff.size() > (size_t)ice::MG_MAX_COLOURS + 1)
+                throw Fail{ICE_ERR_UNSUPPORTED, "too many multigrid colours"};
+        // the coarse levels one workgroup holds in LDS (of its 160 KB, 8 for
+        // partial sums)
+        std::vector<int> n_of;
+        for (const MGLevel& L : mg) n_of.push_back(L.n);
+        tail_level = (int)mg.size() - 1;
+        while (tail_level > 0 &&
+               ice::mg_tail_bytes((int)mg.size() - tail_level + 1, n_of.data() + tail_level - 1, neq) <= 148 * 1024)
+            --tail_level;
+        tail.nlev = (int)mg.size() - tail_level;
+        for (int l = 0; l < tail.nlev; ++l) tail.lev[l] = cells(tail_level + l);
+        fine_ap = alloc<float>((size_t)nelem * nslots * bs * neq);
+        fine_fused = ice::mg_fine_covers(bs, neq, J16 ? 2 : 4);
         coarse_n = mg.back().n * neq;
         if (coarse_n <= 1024) coarse_inv = alloc<double>((size_t)coarse_n * coarse_n);
     }
@@ -415,15 +462,13 @@ struct ice_newton {
     void factor_mg(hipStream_t st) {
         for (size_t l = 0; l < mg.size(); ++l) {
             MGLevel& L = mg[l];
-            if (l == 0)
-                NT_LAUNCH(ice::mg_galerkin_p0(nelem, nslots, nbasis, neq, J64, L.A64, st));
-            else
+            if (l > 0)  // (level 0: formed with the block copies)
                 NT_LAUNCH(ice::mg_galerkin_agg(L.n, nslots, neq, L.children, mg[l - 1].cols, mg[l - 1].parent,
                                                mg[l - 1].A64, L.A64, st));
-            NT_LAUNCH(ice::convert_transpose_fp32((size_t)L.n * nslots, neq, L.A64, L.A32, st));
-            NT_LAUNCH(ice::block_inverse<float>(L.n, nslots, neq, L.A64, L.Dinv, nsing, true, st));
+            NT_LAUNCH(ice::block_inverse<float>(L.n, nslots, neq, L.A64, mg_d, nsing, true, st));
+            NT_LAUNCH(ice::mg_pack(L.n, nslots, neq, L.A64, mg_d, L.A32, L.Dinv, st));
         }
-        coarse_direct = factor_coarse(st);
+        tail.inv = factor_coarse(st) ? coarse_inv : nullptr;
     }
 
     // fine-level V-cycle: SGS, coarse correction through the element
@@ -436,11 +481,19 @@ struct ice_newton {
             else NT_LAUNCH((ice::bsrT_apply<float, double>(nelem, nslots, bs, cols, J32, x, v, mg_r, st)));
         };
         apply_sgs_fine(v, out, st);
-        fine_residual(out);
-        NT_LAUNCH(ice::mg_restrict_nodes(nelem, nbasis, neq, mg_r, mg[0].b, st));
+        if (fine_fused) {
+            if (J16)
+                NT_LAUNCH(ice::mg_fine_residual<_Float16>(nelem, nslots, bs, neq, cols, ecolor, J16, out, v, mg_r,
+                                                          mg[0].b, st));
+            else
+                NT_LAUNCH(ice::mg_fine_residual<float>(nelem, nslots, bs, neq, cols, ecolor, J32, out, v, mg_r,
+                                                       mg[0].b, st));
+        } else {
+            fine_residual(out);
+            NT_LAUNCH(ice::mg_restrict_nodes(nelem, nbasis, neq, mg_r, mg[0].b, st));
+        }
         vcycle(0, mg[0].b, mg[0].x, st);
-        NT_LAUNCH(ice::mg_prolong_nodes(nelem, nbasis, neq, mg[0].x, out, st));
-        fine_residual(out);
+        NT_LAUNCH(ice::mg_fine_correct(nelem, nslots, bs, neq, cols, fine_ap, mg[0].x, out, mg_r, st));
         apply_sgs_fine(mg_r, mg_t, st);
         NT_LAUNCH(ice::launch_axpby2(n, 1.0, mg_t, 1.0, out, st));
     }
@@ -454,7 +507,8 @@ struct ice_newton {
             return;
         }
         if (fp32()) {
-            NT_LAUNCH(ice::convert_transpose_blocks((size_t)nelem * nslots, bs, J64, J32, J16, st));
+            NT_LAUNCH(ice::convert_transpose_blocks((size_t)nelem * nslots, bs, neq, J64, J32, J16, fine_ap,
+                                                    fine_ap ? mg[0].A64 : nullptr, st));
             NT_LAUNCH(ice::block_inverse<float>(nelem, nslots, bs, J64, (float*)Dinv, nsing, true, st));
         } else {
             NT_LAUNCH(ice::block_inverse<double>(nelem, nslots, bs, J64, (double*)Dinv, nsing, false, st));
@@ -488,14 +542,12 @@ struct ice_newton {
                 apply_A(z, Vj(k + 1), st);
                 double* w = Vj(k + 1);
                 NT_LAUNCH(ice::launch_mdot(n, k + 1, V, n, w, part, npart, h1, st));
+                NT_LAUNCH(ice::launch_maxpy_norm(n, k + 1, V, n, h1, w, part, st));
                 if (opt.gmres_cgs_refine) {
-                    NT_LAUNCH(ice::launch_maxpy_norm(n, k + 1, V, n, h1, w, part, nullptr, st));
                     NT_LAUNCH(ice::launch_mdot(n, k + 1, V, n, w, part, npart, h2, st));
-                    NT_LAUNCH(ice::launch_maxpy_norm(n, k + 1, V, n, h2, w, part, h2 + k + 1, st));
-                } else {
-                    NT_LAUNCH(ice::launch_maxpy_norm(n, k + 1, V, n, h1, w, part, h2 + k + 1, st));
+                    NT_LAUNCH(ice::launch_maxpy_norm(n, k + 1, V, n, h2, w, part, st));
                 }
-                NT_LAUNCH(ice::launch_arnoldi(k, m, h1, h2, opt.gmres_cgs_refine, sc, st));
+                NT_LAUNCH(ice::launch_arnoldi(n, k, m, h1, h2, opt.gmres_cgs_refine, part, sc, st));
                 NT_LAUNCH(ice::launch_scale(n, hn, 1, w, st));
                 ++k;
                 ++total;
