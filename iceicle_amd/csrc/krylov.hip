@@ -7,6 +7,7 @@
 #include <algorithm>
 
 #include "kernels.h"
+#include "line_small.h"
 
 namespace ice {
 
@@ -358,187 +359,6 @@ __global__ __launch_bounds__(64) void line_solve_kernel(int nelem, int nslots, i
     }
 }
 
-// The same factorisation and solve for small blocks (bs <= 5, e.g. scalar
-// 1D problems) by a single lane holding everything in registers: the chain
-// is a sequence of dependent steps, and without LDS round trips and barriers
-// each step is a few hundred register operations.  The next element's blocks
-// are loaded a step ahead.  Gauss-Jordan on [S | I] with partial pivoting
-// (largest |S[i][k]|, lowest row on ties) by selects, so no register array
-// is indexed at run time.
-template <int BS>
-__global__ __launch_bounds__(64) void line_factor_small_kernel(int nelem, int nslots, const double* __restrict__ J,
-                                                               double* __restrict__ Sinv, double* __restrict__ W,
-                                                               int* __restrict__ nsingular) {
-    if (threadIdx.x != 0) return;
-    constexpr int BB = BS * BS;
-    double Wp[BB] = {};
-    double cD[BB], cL[BB], cU[BB], nD[BB], nL[BB], nU[BB];
-    auto load = [&](int e, double* d, double* l, double* u) {
-        const double* Je = J + (size_t)e * nslots * BB;
-#pragma unroll
-        for (int k = 0; k < BB; ++k) {
-            d[k] = Je[k];
-            l[k] = Je[BB + k];
-            u[k] = Je[2 * BB + k];
-        }
-    };
-    load(0, cD, cL, cU);
-    for (int e = 0; e < nelem; ++e) {
-        if (e + 1 < nelem) load(e + 1, nD, nL, nU);
-        double A[BS][2 * BS];
-#pragma unroll
-        for (int i = 0; i < BS; ++i)
-#pragma unroll
-            for (int c = 0; c < BS; ++c) {
-                double sacc = cD[i * BS + c];
-                if (e > 0)
-#pragma unroll
-                    for (int k = 0; k < BS; ++k) sacc -= cL[i * BS + k] * Wp[k * BS + c];
-                A[i][c] = sacc;
-                A[i][BS + c] = (i == c) ? 1.0 : 0.0;
-            }
-        bool bad = false;
-#pragma unroll
-        for (int k = 0; k < BS; ++k) {
-            int piv = k;
-            double best = fabs(A[k][k]);
-#pragma unroll
-            for (int i = k + 1; i < BS; ++i) {
-                const double a = fabs(A[i][k]);
-                if (a > best) { best = a; piv = i; }
-            }
-            if (!(best > 0.0)) bad = true;
-#pragma unroll
-            for (int i = k + 1; i < BS; ++i)
-#pragma unroll
-                for (int c = 0; c < 2 * BS; ++c) {
-                    const double tk = A[k][c], ti = A[i][c];
-                    A[k][c] = (piv == i) ? ti : tk;
-                    A[i][c] = (piv == i) ? tk : ti;
-                }
-            const double ip = 1.0 / A[k][k];
-#pragma unroll
-            for (int c = 0; c < 2 * BS; ++c) A[k][c] *= ip;
-#pragma unroll
-            for (int i = 0; i < BS; ++i) {
-                if (i == k) continue;
-                const double f = A[i][k];
-#pragma unroll
-                for (int c = 0; c < 2 * BS; ++c) A[i][c] -= f * A[k][c];
-            }
-        }
-        if (bad) {
-#pragma unroll
-            for (int i = 0; i < BS; ++i)
-#pragma unroll
-                for (int c = 0; c < BS; ++c) A[i][BS + c] = (i == c) ? 1.0 : 0.0;
-            atomicAdd(nsingular, 1);
-        }
-        double* So = Sinv + (size_t)e * BB;
-#pragma unroll
-        for (int i = 0; i < BS; ++i)
-#pragma unroll
-            for (int c = 0; c < BS; ++c) So[i * BS + c] = A[i][BS + c];
-        if (e + 1 < nelem) {
-            double* Wo = W + (size_t)e * BB;
-#pragma unroll
-            for (int i = 0; i < BS; ++i)
-#pragma unroll
-                for (int c = 0; c < BS; ++c) {
-                    double sacc = 0.0;
-#pragma unroll
-                    for (int k = 0; k < BS; ++k) sacc += A[i][BS + k] * cU[k * BS + c];
-                    Wp[i * BS + c] = sacc;
-                    Wo[i * BS + c] = sacc;
-                }
-#pragma unroll
-            for (int k = 0; k < BB; ++k) {
-                cD[k] = nD[k];
-                cL[k] = nL[k];
-                cU[k] = nU[k];
-            }
-        }
-    }
-}
-
-template <int BS>
-__global__ __launch_bounds__(64) void line_solve_small_kernel(int nelem, int nslots, const double* __restrict__ J,
-                                                              const double* __restrict__ Sinv,
-                                                              const double* __restrict__ W, const double* __restrict__ b,
-                                                              double* __restrict__ x) {
-    if (threadIdx.x != 0) return;
-    constexpr int BB = BS * BS;
-    double yp[BS] = {};
-    double cL[BB], cS[BB], cb[BS], nL[BB], nS[BB], nb[BS];
-    auto load = [&](int e, double* l, double* si, double* bv) {
-        const double* L = J + ((size_t)e * nslots + 1) * BB;
-#pragma unroll
-        for (int k = 0; k < BB; ++k) {
-            l[k] = L[k];
-            si[k] = Sinv[(size_t)e * BB + k];
-        }
-#pragma unroll
-        for (int k = 0; k < BS; ++k) bv[k] = b[(size_t)e * BS + k];
-    };
-    load(0, cL, cS, cb);
-    for (int e = 0; e < nelem; ++e) {
-        if (e + 1 < nelem) load(e + 1, nL, nS, nb);
-        double t[BS];
-#pragma unroll
-        for (int i = 0; i < BS; ++i) {
-            double sacc = cb[i];
-            if (e > 0)
-#pragma unroll
-                for (int k = 0; k < BS; ++k) sacc -= cL[i * BS + k] * yp[k];
-            t[i] = sacc;
-        }
-#pragma unroll
-        for (int i = 0; i < BS; ++i) {
-            double sacc = 0.0;
-#pragma unroll
-            for (int k = 0; k < BS; ++k) sacc += cS[i * BS + k] * t[k];
-            yp[i] = sacc;
-            x[(size_t)e * BS + i] = sacc;
-        }
-#pragma unroll
-        for (int k = 0; k < BB; ++k) {
-            cL[k] = nL[k];
-            cS[k] = nS[k];
-        }
-#pragma unroll
-        for (int k = 0; k < BS; ++k) cb[k] = nb[k];
-    }
-    // backward: x_e = y_e - W_e x_{e+1}; yp holds x_{n-1}
-    double cW[BB], cy[BS], nW[BB], ny[BS];
-    auto loadb = [&](int e, double* w, double* yv) {
-#pragma unroll
-        for (int k = 0; k < BB; ++k) w[k] = W[(size_t)e * BB + k];
-#pragma unroll
-        for (int k = 0; k < BS; ++k) yv[k] = x[(size_t)e * BS + k];
-    };
-    if (nelem >= 2) loadb(nelem - 2, cW, cy);
-    for (int e = nelem - 2; e >= 0; --e) {
-        if (e >= 1) loadb(e - 1, nW, ny);
-        double xe[BS];
-#pragma unroll
-        for (int i = 0; i < BS; ++i) {
-            double sacc = cy[i];
-#pragma unroll
-            for (int k = 0; k < BS; ++k) sacc -= cW[i * BS + k] * yp[k];
-            xe[i] = sacc;
-        }
-#pragma unroll
-        for (int i = 0; i < BS; ++i) {
-            yp[i] = xe[i];
-            x[(size_t)e * BS + i] = xe[i];
-        }
-#pragma unroll
-        for (int k = 0; k < BB; ++k) cW[k] = nW[k];
-#pragma unroll
-        for (int k = 0; k < BS; ++k) cy[k] = ny[k];
-    }
-}
-
 // y[e] = D[e] x[e] for dense bs x bs blocks (block-Jacobi application), one
 // block row per lane group as in bsr_kernel
 template <class T, class V>
@@ -594,30 +414,16 @@ int line_factor(int nelem, int nslots, int bs, const double* J, double* Sinv, do
                 hipStream_t st) {
     const size_t sh = 8 * (size_t)bs * bs * sizeof(double) + (size_t)bs * sizeof(int);
     if (bs > 16 || nslots < 3 || nelem < 1) return -1;
-    switch (bs) {
-    case 1: line_factor_small_kernel<1><<<1, 64, 0, st>>>(nelem, nslots, J, Sinv, W, nsingular); break;
-    case 2: line_factor_small_kernel<2><<<1, 64, 0, st>>>(nelem, nslots, J, Sinv, W, nsingular); break;
-    case 3: line_factor_small_kernel<3><<<1, 64, 0, st>>>(nelem, nslots, J, Sinv, W, nsingular); break;
-    case 4: line_factor_small_kernel<4><<<1, 64, 0, st>>>(nelem, nslots, J, Sinv, W, nsingular); break;
-    case 5: line_factor_small_kernel<5><<<1, 64, 0, st>>>(nelem, nslots, J, Sinv, W, nsingular); break;
-    default: line_factor_kernel<<<1, 64, sh, st>>>(nelem, nslots, bs, J, Sinv, W, nsingular); break;
-    }
+    if (bs <= LINE_SMALL) return line_small_factor(nelem, nslots, bs, J, Sinv, W, nsingular, st);
+    line_factor_kernel<<<1, 64, sh, st>>>(nelem, nslots, bs, J, Sinv, W, nsingular);
     return (int)hipGetLastError();
 }
 
 int line_solve(int nelem, int nslots, int bs, const double* J, const double* Sinv, const double* W, const double* b,
                double* x, hipStream_t st) {
     if (bs > 16 || nslots < 3 || nelem < 1) return -1;
-    switch (bs) {
-    case 1: line_solve_small_kernel<1><<<1, 64, 0, st>>>(nelem, nslots, J, Sinv, W, b, x); break;
-    case 2: line_solve_small_kernel<2><<<1, 64, 0, st>>>(nelem, nslots, J, Sinv, W, b, x); break;
-    case 3: line_solve_small_kernel<3><<<1, 64, 0, st>>>(nelem, nslots, J, Sinv, W, b, x); break;
-    case 4: line_solve_small_kernel<4><<<1, 64, 0, st>>>(nelem, nslots, J, Sinv, W, b, x); break;
-    case 5: line_solve_small_kernel<5><<<1, 64, 0, st>>>(nelem, nslots, J, Sinv, W, b, x); break;
-    default:
-        line_solve_kernel<<<1, 64, 2 * (size_t)bs * sizeof(double), st>>>(nelem, nslots, bs, J, Sinv, W, b, x);
-        break;
-    }
+    if (bs <= LINE_SMALL) return line_small_solve(nelem, nslots, bs, J, Sinv, W, b, x, st);
+    line_solve_kernel<<<1, 64, 2 * (size_t)bs * sizeof(double), st>>>(nelem, nslots, bs, J, Sinv, W, b, x);
     return (int)hipGetLastError();
 }
 

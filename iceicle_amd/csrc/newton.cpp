@@ -21,6 +21,7 @@
 #include "engine.h"
 #include "kernels.h"
 #include "linesearch.h"
+#include "line_small.h"
 #include "mg.h"
 
 namespace ice {
@@ -705,7 +706,8 @@ int ice_newton_create(ice_disc* d, const ice_newton_opts* opts, ice_newton** out
             if (!chain)
                 throw Fail{ICE_ERR_UNSUPPORTED, "the line preconditioner needs a non-periodic 1D mesh"};
             s->line_Sinv = s->alloc<double>((size_t)s->nelem * s->bs * s->bs);
-            s->line_W = s->alloc<double>((size_t)s->nelem * s->bs * s->bs);
+            s->line_W = s->alloc<double>(s->bs <= ice::LINE_SMALL ? ice::line_small_work(s->nelem, s->bs)
+                                                                  : (size_t)s->nelem * s->bs * s->bs);
         } else if (o.preconditioner != ICE_PC_BLOCK_JACOBI) {
             s->colour();
         }
