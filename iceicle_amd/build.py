@@ -16,7 +16,7 @@ OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libiceicle_amd.so")
 
 SOURCES = ["mesh.cpp", "engine.cpp", "residual.hip", "residual_wave2d_burgers.hip", "residual_wave2d_ns.hip",
-           "residual_wave2d_euler.hip", "residual_wave3d.hip", "stepper.hip", "jacobian.hip", "jacobian_rows.hip", "krylov.hip", "line_small.hip", "mg.hip", "newton.cpp",
+           "residual_wave2d_euler.hip", "residual_wave3d.hip", "residual_lane2d.hip", "stepper.hip", "jacobian.hip", "jacobian_rows.hip", "krylov.hip", "line_small.hip", "mg.hip", "newton.cpp",
            "mlp.hip", "noalloc.hip", "mdg.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -121,10 +121,21 @@ int launch_widen(size_t n, const float* x, double* y, hipStream_t st);  // y = (
 int launch_step_begin(StepState* s, unsigned long long* wave, const StepControl& c, hipStream_t st);
 int launch_step_end(StepState* s, hipStream_t st);
 
-// One-launch residuals (residual_wave2d.h, residual_wave3d.h): 2D P1-P3
-// without DDGIC vectors, 3D Euler P2 and P3.
+// One-launch residuals without DDGIC vectors (residual_wave2d.h,
+// residual_lane2d.h, residual_wave3d.h): 2D P1-P3, scalar 2D P4, 3D Euler P2
+// and P3.
 inline bool wave_covers(int ndim, int p, int flux, const DiscDev& dd) {
-    return (ndim == 2 && p <= 3 && !dd.Pic) || (ndim == 3 && flux == ICE_FLUX_EULER && (p == 2 || p == 3));
+    return (ndim == 2 && (p <= 3 || flux == ICE_FLUX_BURGERS) && !dd.Pic) ||
+           (ndim == 3 && flux == ICE_FLUX_EULER && (p == 2 || p == 3));
+}
+// The scalar 2D ones by lanes, from the element count where a step of 3
+// stages is faster than with matrix instructions, a wave of which is 4
+// elements to its 16 but shorter: P1 80^2 20.8 us for 21.7 (64^2 20.8 for
+// 18.6), P2 96^2 26.5 for 26.9 (80^2 25.9 for 22.2), P3 160^2 43.3 for 44.5
+// (128^2 34.2 for 30.9).  P4 has only this one.
+inline bool lane2d_covers(int p, int flux, int nelem) {
+    constexpr int from[4] = {6400, 9216, 25600, 0};
+    return flux == ICE_FLUX_BURGERS && nelem >= from[p - 1];
 }
 // Their stage form: K = M^-1 R(U) and the stage combination cb, U not
 // aliasing cb.out.

@@ -2155,6 +2155,7 @@ int launch_residual(const DevSpace& S, const typename PH::Params& ph, const Disc
     int F(int p, const DevSpace& S, const PhysT<float>& ph, const DiscDev& dd, const float* U, double* R, float* K, \
           const StageComb<float>& cb, hipStream_t st);
 ICE_WAVE_DECL(wave2d_burgers)
+ICE_WAVE_DECL(lane2d_burgers)
 ICE_WAVE_DECL(wave2d_ns)
 ICE_WAVE_DECL(wave2d_euler)
 ICE_WAVE_DECL(wave3d_euler)
@@ -2163,6 +2164,7 @@ ICE_WAVE_DECL(wave3d_euler)
 template <class R, class... A>
 int wave_residual(int flux, int p, const DevSpace& S, const PhysT<R>& ph, const DiscDev& dd, A... a) {
     if (S.ndim == 3) return wave3d_euler(p, S, ph, dd, a...);
+    if (lane2d_covers(p, flux, S.nelem)) return lane2d_burgers(p, S, ph, dd, a...);
     if (flux == ICE_FLUX_BURGERS) return wave2d_burgers(p, S, ph, dd, a...);
     if (flux == ICE_FLUX_NAVIER_STOKES) return wave2d_ns(p, S, ph, dd, a...);
     if (flux == ICE_FLUX_EULER) return wave2d_euler(p, S, ph, dd, a...);
@@ -2193,7 +2195,7 @@ int residual_stage(int ndim, int p, int flux, const DevSpace& S, const PhysParam
 template <class PH, int D, class UT = double>
 int dispatch_order(int p, const DevSpace& S, const typename PH::Params& ph, const DiscDev& dd, const UT* U,
                    double* R, hipStream_t st, hipEvent_t* ev) {
-    // P1-P3 in 2D come here with the DDGIC lifting vectors only, 3D fluxes
+    // P1-P3 in 2D and the scalar P4 come here with the DDGIC lifting vectors only, 3D fluxes
     // without a gradient not with P2 and P3 (wave_covers)
     constexpr bool EULER3 = D == 3 && !TraceRec<PH, D>::NEED_GRAD;
     if (p == 4) return launch_residual<D, 4, PH, UT>(S, ph, dd, U, R, st, ev);

@@ -1,0 +1,58 @@
+"""Scalar 2D residual by lanes, taken for many elements, against the wave
+kernel taken for few (P4, which the lanes always take: in other places of a
+wave): a space of copies of one small mesh has the small mesh's residual in
+every copy.
+
+The two differ in the order of sums only: FP64 within 1e-12 of the largest
+entry, and so with FP32 fluxes but for an FP32 rounding of the point values
+(1e-5); a stage likewise."""
+import numpy as np
+import pytest
+
+from iceicle_amd import abi
+from tests import cases
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+D, P, N = "DIRICHLET", "PERIODIC", "NEUMANN"
+MIN = {1: 6400, 2: 9216, 3: 25600, 4: 1000}  # elements from which the lanes are taken
+
+
+def _spaces(order, nel, bc, copies):
+    from iceicle_amd import engine
+    m = abi.mesh_desc(2, nel, [0.0, 0.0], [1.0, 0.8], bc, bcflag=[0, 1, 1, 0], periodic_mode=abi.PERIODIC_COUPLED)
+    m = abi.mesh_desc(2, nel, [0.0, 0.0], [1.0, 0.8], bc, bcflag=[0, 1, 1, 0], periodic_mode=abi.PERIODIC_COUPLED,
+                      coord=cases.perturbed_coords(m, 0.1, 3))
+    return [(engine.FESpace([m] * k, order), k) for k in (1, copies)]
+
+
+@pytest.mark.parametrize("order", [1, 2, 3, 4])
+@pytest.mark.parametrize("nel,bc", [([13, 9], [P, P, P, P]), ([8, 16], [D, N, N, D]), ([5, 7], [P, D, P, N])])
+def test_copies(order, nel, bc):
+    from iceicle_amd import engine
+    ne = nel[0] * nel[1]
+    prm = cases.burgers_params(2, mu=0.02, a=(0.3, -0.2, 0.0), b=(1.0, 0.7, 0.0))
+    rng = np.random.default_rng(order)
+    u1 = rng.uniform(-1.0, 1.0, ne * (order + 1) ** 2)
+    out = {}
+    for space, k in _spaces(order, nel, bc, -(-MIN[order] // ne)):
+        assert (space.nelem >= MIN[order]) == (k > 1)
+        disc = engine.ConservationLawDDG(space, prm)
+        u = torch.from_numpy(np.tile(u1, k)).cuda()
+        r = torch.full_like(u, float("nan"))
+        rm = torch.full_like(u, float("nan"))
+        engine.form_residual(space, disc, u, r)
+        engine.form_residual(space, disc, u, rm, precision="mixed")
+        v = u.clone()
+        st = engine.ExplicitStepper(disc, abi.stepper_desc(abi.STEP_RK3_SSP, dt=1e-3, ntime=2))
+        w = u.float()
+        for _ in range(2):
+            st.step(v)
+            st.step(w)
+        out[k] = [x.view(k, -1).cpu().numpy() for x in (r, rm, v, w)]
+    (small, big) = out[1], out[max(out)]
+    for a, b, tol in zip(small, big, (1e-12, 1e-5, 1e-12, 1e-5)):
+        err = np.abs(b - a).max() / np.abs(a).max()
+        print(f"P{order} {nel} {bc}: {err:.1e}", flush=True)
+        assert err <= tol
