@@ -548,11 +548,11 @@ __global__ __launch_bounds__(256) void maxpy_norm_kernel(size_t n, int nv, const
     if (threadIdx.x == 0 && part) part[blockIdx.x] = s;
 }
 
-// x += sum_j y[j] V_j
+// x = sum_j y[j] V_j
 __global__ __launch_bounds__(256) void combine_kernel(size_t n, int nv, const double* __restrict__ V, size_t ldv,
                                                       const double* __restrict__ y, double* __restrict__ x) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        double s = x[i];
+        double s = 0.0;
         for (int j = 0; j < nv; ++j) s += y[j] * V[(size_t)j * ldv + i];
         x[i] = s;
     }
@@ -581,7 +581,7 @@ __global__ void axpby_kernel2(size_t n, double a, const double* __restrict__ x, 
 __global__ __launch_bounds__(256) void arnoldi_kernel(int k, int m, const double* __restrict__ h1,
                                                       const double* __restrict__ h2, int refine,
                                                       const double* __restrict__ part, int nblk,
-                                                      double* __restrict__ sc) {
+                                                      double* __restrict__ sc, double* __restrict__ host) {
     extern __shared__ double sh[];  // column [m + 1], cs [m], sn [m]
     __shared__ double red[4];
     double* H = sc;                       // (m+1) x m, column-major: H[j + (m+1) k]
@@ -617,7 +617,7 @@ __global__ __launch_bounds__(256) void arnoldi_kernel(int k, int m, const double
         col[k + 1] = 0.0;
         g[k + 1] = -s * g[k];
         g[k] = c * g[k];
-        hn[1] = fabs(g[k + 1]);
+        hn[1] = *host = fabs(g[k + 1]);
     }
     __syncthreads();
     for (int j = threadIdx.x; j <= k; j += blockDim.x) col[j] = scol[j];
@@ -637,7 +637,8 @@ __global__ void hessenberg_solve_kernel(int k, int m, const double* __restrict__
 }
 
 // g = (beta, 0, ...), beta = sqrt(*nrm2)
-__global__ void gmres_init_kernel(int m, const double* __restrict__ nrm2, double* __restrict__ sc) {
+__global__ void gmres_init_kernel(int m, const double* __restrict__ nrm2, double* __restrict__ sc,
+                                  double* __restrict__ host) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     double* g = sc + (size_t)(m + 1) * m + 2 * m;
     g[0] = sqrt(fmax(*nrm2, 0.0));
@@ -645,7 +646,35 @@ __global__ void gmres_init_kernel(int m, const double* __restrict__ nrm2, double
     double* hn = g + m + 1;
     hn[0] = g[0];
     hn[1] = g[0];
+    *host = g[0];
 }
+
+// w.w (or the sum of its partial sums) by one workgroup, also stored to
+// pinned host memory: the host reads its scalars after a stream
+// synchronization without a copy on the way.  Up to NORM_ONE entries the two
+// launches and the copy of 2-5 us each become one launch of 2.4 us (1D layer
+// solve of 1024 unknowns, 31 norms and 4 linear solves: 3.6 -> 2.3 ms with the
+// grids below); beyond, one workgroup would be the longer.
+constexpr size_t NORM_ONE = 16384;
+template <bool SQUARE>
+__device__ __forceinline__ void norm2_one(int n, const double* __restrict__ w, double* __restrict__ out,
+                                          double* __restrict__ host) {
+    __shared__ double red[16];
+    double s = 0.0;
+#pragma unroll 8
+    for (int i = threadIdx.x; i < n; i += 1024) s += SQUARE ? w[i] * w[i] : w[i];
+    s = block_sum(s, red);
+    if (threadIdx.x == 0) *out = *host = s;
+}
+__global__ __launch_bounds__(1024) void norm2_kernel(int n, const double* w, double* out, double* host) {
+    norm2_one<true>(n, w, out, host);
+}
+__global__ __launch_bounds__(1024) void norm2_kernel_reduce(int n, const double* part, double* out, double* host) {
+    norm2_one<false>(n, part, out, host);
+}
+
+// workgroups of an elementwise kernel
+unsigned elem_grid(size_t n) { return (unsigned)std::min<size_t>((n + 255) / 256, 2048); }
 
 int vec_grid(size_t n) { return (int)((n + 256 * VEC_EPT - 1) / (256 * VEC_EPT)); }
 
@@ -658,8 +687,9 @@ int gmres_partials(size_t n) { return maxpy_grid(n); }
 int launch_mdot(size_t n, int nv, const double* V, size_t ldv, const double* w, double* part, int npart, double* out,
                 hipStream_t st) {
     const int nb = vec_grid(n);
+    if (nb == 1) part = out;  // a single chunk's sums are the result
     mdot_partial_kernel<<<dim3(nb, nv / MDOT_VECS + 1), 256, 0, st>>>(n, nv, V, ldv, w, part, npart);
-    reduce_partials_kernel<<<nv + 1, 256, 0, st>>>(nb, part, npart, out);
+    if (nb > 1) reduce_partials_kernel<<<nv + 1, 256, 0, st>>>(nb, part, npart, out);
     return (int)hipGetLastError();
 }
 
@@ -669,28 +699,36 @@ int launch_maxpy_norm(size_t n, int nv, const double* V, size_t ldv, const doubl
     return (int)hipGetLastError();
 }
 
-int launch_norm2(size_t n, const double* w, double* part, double* out, hipStream_t st) {
-    return launch_mdot(n, 0, nullptr, 0, w, part, 1, out, st);
+int launch_norm2(size_t n, const double* w, double* part, double* out, double* host, hipStream_t st) {
+    if (n <= NORM_ONE) {
+        norm2_kernel<<<1, 1024, 0, st>>>((int)n, w, out, host);
+        return (int)hipGetLastError();
+    }
+    const int nb = vec_grid(n);
+    mdot_partial_kernel<<<dim3(nb, 1), 256, 0, st>>>(n, 0, nullptr, 0, w, part, 1);
+    norm2_kernel_reduce<<<1, 1024, 0, st>>>(nb, part, out, host);
+    return (int)hipGetLastError();
 }
 
 int launch_combine(size_t n, int nv, const double* V, size_t ldv, const double* y, double* x, hipStream_t st) {
-    combine_kernel<<<2048, 256, 0, st>>>(n, nv, V, ldv, y, x);
+    combine_kernel<<<elem_grid(n), 256, 0, st>>>(n, nv, V, ldv, y, x);
     return (int)hipGetLastError();
 }
 
 int launch_scale(size_t n, const double* s, int inv, double* x, hipStream_t st) {
-    scale_kernel<<<2048, 256, 0, st>>>(n, s, inv, x);
+    scale_kernel<<<elem_grid(n), 256, 0, st>>>(n, s, inv, x);
     return (int)hipGetLastError();
 }
 
 int launch_axpby2(size_t n, double a, const double* x, double b, double* y, hipStream_t st) {
-    axpby_kernel2<<<2048, 256, 0, st>>>(n, a, x, b, y);
+    axpby_kernel2<<<elem_grid(n), 256, 0, st>>>(n, a, x, b, y);
     return (int)hipGetLastError();
 }
 
 int launch_arnoldi(size_t n, int k, int m, const double* h1, const double* h2, int refine, const double* part,
-                   double* sc, hipStream_t st) {
-    arnoldi_kernel<<<1, 256, (size_t)(3 * m + 1) * sizeof(double), st>>>(k, m, h1, h2, refine, part, maxpy_grid(n), sc);
+                   double* sc, double* host, hipStream_t st) {
+    arnoldi_kernel<<<1, 256, (size_t)(3 * m + 1) * sizeof(double), st>>>(k, m, h1, h2, refine, part, maxpy_grid(n), sc,
+                                                                         host);
     return (int)hipGetLastError();
 }
 
@@ -699,8 +737,8 @@ int launch_hessenberg_solve(int k, int m, const double* sc, double* y, hipStream
     return (int)hipGetLastError();
 }
 
-int launch_gmres_init(int m, const double* nrm2, double* sc, hipStream_t st) {
-    gmres_init_kernel<<<1, 64, 0, st>>>(m, nrm2, sc);
+int launch_gmres_init(int m, const double* nrm2, double* sc, double* host, hipStream_t st) {
+    gmres_init_kernel<<<1, 64, 0, st>>>(m, nrm2, sc, host);
     return (int)hipGetLastError();
 }
 

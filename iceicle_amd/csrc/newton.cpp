@@ -55,14 +55,14 @@ int launch_mdot(size_t n, int nv, const double* V, size_t ldv, const double* w, 
                 hipStream_t st);
 int launch_maxpy_norm(size_t n, int nv, const double* V, size_t ldv, const double* h, double* w, double* part,
                       hipStream_t st);
-int launch_norm2(size_t n, const double* w, double* part, double* out, hipStream_t st);
+int launch_norm2(size_t n, const double* w, double* part, double* out, double* host, hipStream_t st);
 int launch_combine(size_t n, int nv, const double* V, size_t ldv, const double* y, double* x, hipStream_t st);
 int launch_scale(size_t n, const double* s, int inv, double* x, hipStream_t st);
 int launch_axpby2(size_t n, double a, const double* x, double b, double* y, hipStream_t st);
 int launch_arnoldi(size_t n, int k, int m, const double* h1, const double* h2, int refine, const double* part,
-                   double* sc, hipStream_t st);
+                   double* sc, double* host, hipStream_t st);
 int launch_hessenberg_solve(int k, int m, const double* sc, double* y, hipStream_t st);
-int launch_gmres_init(int m, const double* nrm2, double* sc, hipStream_t st);
+int launch_gmres_init(int m, const double* nrm2, double* sc, double* host, hipStream_t st);
 template <class T, class V>
 int sgs_sweep(bool forward, int nrows, const int* elems, const int* ecolor, int c, int nslots, int bs,
               const int* cols, const T* J, const T* Dinv, const V* r, V* y, hipStream_t st);
@@ -171,14 +171,14 @@ struct ice_newton {
     bool fp32() const { return opt.jacobian_precision == ICE_PREC_FP32; }
     double* Vj(int j) const { return V + (size_t)j * n; }
 
-    double read_scalar(const double* d, hipStream_t st) {
-        NT_HIP(hipMemcpyAsync(host, d, sizeof(double), hipMemcpyDeviceToHost, st));
+    // the scalar that the last norm, gmres_init or arnoldi launch stored to host[0]
+    double read_scalar(hipStream_t st) {
         NT_HIP(hipStreamSynchronize(st));
         return host[0];
     }
     double norm(const double* v, hipStream_t st) {
-        NT_LAUNCH(ice::launch_norm2(n, v, part, h1, st));
-        return std::sqrt(std::max(read_scalar(h1, st), 0.0));
+        NT_LAUNCH(ice::launch_norm2(n, v, part, h1, host, st));
+        return std::sqrt(std::max(read_scalar(st), 0.0));
     }
 
     // Krylov operator w = A z and preconditioner z = M^-1 v
@@ -525,10 +525,10 @@ struct ice_newton {
     int gmres(const double* b, double* x, double rtol, int maxit, hipStream_t st, double* est) {
         int total = 0;
         NT_HIP(hipMemcpyAsync(Vj(0), b, n * sizeof(double), hipMemcpyDeviceToDevice, st));
-        NT_LAUNCH(ice::launch_norm2(n, Vj(0), part, h1, st));
-        NT_LAUNCH(ice::launch_gmres_init(m, h1, sc, st));
+        NT_LAUNCH(ice::launch_norm2(n, Vj(0), part, h1, host, st));
+        NT_LAUNCH(ice::launch_gmres_init(m, h1, sc, host, st));
         const double* beta_d = sc + (size_t)(m + 1) * m + 2 * m;  // g[0]
-        const double beta0 = read_scalar(beta_d, st);
+        const double beta0 = read_scalar(st);
         *est = 0.0;
         if (!(beta0 > 0.0)) return 0;
         const double target = rtol * beta0;
@@ -548,16 +548,15 @@ struct ice_newton {
                     NT_LAUNCH(ice::launch_mdot(n, k + 1, V, n, w, part, npart, h2, st));
                     NT_LAUNCH(ice::launch_maxpy_norm(n, k + 1, V, n, h2, w, part, st));
                 }
-                NT_LAUNCH(ice::launch_arnoldi(n, k, m, h1, h2, opt.gmres_cgs_refine, part, sc, st));
+                NT_LAUNCH(ice::launch_arnoldi(n, k, m, h1, h2, opt.gmres_cgs_refine, part, sc, host, st));
                 NT_LAUNCH(ice::launch_scale(n, hn, 1, w, st));
                 ++k;
                 ++total;
-                r = read_scalar(hn + 1, st);
+                r = read_scalar(st);
                 if (!(r > target) || total >= maxit || !std::isfinite(r)) break;
             }
             // x += M^-1 V_k y_k
             NT_LAUNCH(ice::launch_hessenberg_solve(k, m, sc, y, st));
-            NT_LAUNCH(ice::launch_axpby2(n, 0.0, t, 0.0, t, st));
             NT_LAUNCH(ice::launch_combine(n, k, V, n, y, t, st));
             apply_M(t, z, st);
             NT_LAUNCH(ice::launch_axpby2(n, 1.0, z, 1.0, x, st));
@@ -567,9 +566,9 @@ struct ice_newton {
             apply_A(x, z, st);
             NT_HIP(hipMemcpyAsync(Vj(0), b, n * sizeof(double), hipMemcpyDeviceToDevice, st));
             NT_LAUNCH(ice::launch_axpby2(n, -1.0, z, 1.0, Vj(0), st));
-            NT_LAUNCH(ice::launch_norm2(n, Vj(0), part, h1, st));
-            NT_LAUNCH(ice::launch_gmres_init(m, h1, sc, st));
-            const double beta = read_scalar(beta_d, st);
+            NT_LAUNCH(ice::launch_norm2(n, Vj(0), part, h1, host, st));
+            NT_LAUNCH(ice::launch_gmres_init(m, h1, sc, host, st));
+            const double beta = read_scalar(st);
             if (!(beta > target)) {
                 *est = beta / beta0;
                 break;

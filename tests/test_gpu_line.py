@@ -1,7 +1,8 @@
 """Line preconditioner (block tridiagonal solve) of 1D problems: cyclic
 reduction with a row a thread and elimination along the chain, at the row
 counts where the number of steps, the threads and the rule between the two
-change, for every small block size.
+change, for every small block size; and a norm's sizes on both sides of one
+workgroup's 16384 entries.
 
 With the preconditioner an exact inverse, J x = b is solved in one iteration
 (two, should the first leave a residual above the tolerance asked); x is held
@@ -18,7 +19,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("order,nelem", [(3, 2), (3, 4), (1, 5), (3, 5), (2, 8), (3, 63), (4, 64), (1, 65), (2, 129), (3, 255),
                                          (3, 256), (4, 257), (3, 300), (2, 511), (4, 512), (3, 513), (4, 1023),
-                                         (1, 1024), (4, 1024), (3, 1025)])
+                                         (1, 1024), (4, 1024), (3, 1025),
+                                         (3, 4096), (3, 4097)])
 def test_line_solve(order, nelem):
     from iceicle_amd import engine
     p = cases.burgers_params(1, mu=0.02, a=(0.5, 0, 0))
