@@ -516,7 +516,8 @@ def batch_leg(ninst=512, reps=20, nsteps=10):
     for k, (sp, dc, uu, rr) in enumerate(singles):
         uu.copy_(bt.instance_state(k))
     ms_single = timed(lambda: [engine.form_residual(sp, dc, uu, rr) for sp, dc, uu, rr in singles], 3)
-    same = all(torch.equal(rr, outs_k) for (sp, dc, uu, rr), outs_k in
+    # (the batch of many elements takes another kernel than one instance: equal to rounding)
+    diff = max(float((rr - outs_k).abs().max() / rr.abs().max()) for (sp, dc, uu, rr), outs_k in
                zip(singles, [r64[bt.index[k][0]][bt.groups[bt.index[k][0]].instance_slice(bt.index[k][1])]
                              for k in range(ninst)]))
     del singles
@@ -559,7 +560,7 @@ def batch_leg(ninst=512, reps=20, nsteps=10):
         "residual_mixed": {"ms": round(ms32, 4), "GDOF_s": round(bt.size / (ms32 * 1e-3) / 1e9, 3),
                            "rel_err_vs_fp64": float(f"{err32:.3e}")},
         "residual_per_instance": {"ms": round(ms_single, 3), "GDOF_s": round(bt.size / (ms_single * 1e-3) / 1e9, 3),
-                                  "bit_identical_to_batched": bool(same)},
+                                  "rel_diff_to_batched": float(f"{diff:.1e}")},
         "rk3_ssp_step_ms": {"eager": round(ms_eager, 4), "graph": round(ms_graph, 4),
                             "graph_concurrent_orders": round(ms_graph_conc, 4), "graph_steps": nsteps},
         "state_finite": finite,
@@ -692,7 +693,7 @@ def main():
         "ms_per_step": round(mixed_ms, 6),
         "rel_err_vs_fp64": float(f"{mixed_err:.3e}"),
         "kernels_ms": {"residual": round(sum(mstage) / mcalls, 6)},
-        "arithmetic": "FP32 interpolation, fluxes and face data; FP64 geometry, source load and output",
+        "arithmetic": "FP32 fluxes; FP64 interpolation, geometry, contractions, source load and output",
     }
 
     def newton_leg(label, **kw):

@@ -147,7 +147,8 @@ int launch_wave_reduce(const double* part, int n, unsigned long long* wave, hipS
 
 int residual_fp64(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                   const double* U, double* R, hipStream_t st, hipEvent_t* ev = nullptr);
-// FP32 interpolation, fluxes and face data with FP64 geometry and output;
+// FP32 fluxes (and, in the three launches, interpolation and face data) with
+// FP64 geometry and output;
 // ndim 2 only (-2 otherwise)
 int residual_mixed(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                    const double* U, double* R, hipStream_t st, hipEvent_t* ev = nullptr);

@@ -308,7 +308,7 @@ def current_stream():
 
 def form_residual(space, disc, u, res, stream=None, precision="fp64"):
     """res <- R(u) on the GPU; precision "fp64" (the reference's arithmetic)
-    or "mixed" (FP32 interpolation and fluxes, FP64 geometry and output, 2D and 3D).
+    or "mixed" (FP32 fluxes, FP64 geometry and output, 2D and 3D).
     u may be an FP32 state (2D and 3D): "mixed" is then the residual FP32
     steps use, "fp64" the FP64 residual of the widened state (the check of an
     FP32 solution against the FP64 discretization).  res is float64."""

@@ -275,9 +275,10 @@ int ice_disc_autotune(ice_disc* disc, const double* u_dev, double* r_dev, int re
 int ice_residual(ice_disc* disc, const double* u_dev, double* res_dev, void* stream);
 
 /* Mixed-precision residual (no reference counterpart; the reference is FP64
- * throughout): the same R(u) with the trace interpolation, the physical and
- * numerical fluxes, the volume contractions and the face data in FP32, and
- * the geometric Jacobians, source load, face lifting sums and R in FP64.
+ * throughout): the same R(u) with the physical and numerical fluxes in FP32,
+ * and the geometric Jacobians, source load, face lifting sums and R in FP64.
+ * Interpolation and volume contractions are FP64 where one launch forms the
+ * residual (ice_disc_set_tile), FP32 elsewhere.
  * ndim = 2 and 3 (ICE_ERR_UNSUPPORTED for ndim = 1).  Expect ~1e-7 of the
  * largest flux terms in absolute error. */
 int ice_residual_mixed(ice_disc* disc, const double* u_dev, double* r_dev, void* stream);
