@@ -204,6 +204,100 @@ __global__ __launch_bounds__(256) void block_inverse_kernel(int nelem, int nslot
     }
 }
 
+// The same for blocks of up to 16 A rows, the block in the workgroup's
+// registers: thread (ti, tj) holds rows ti + 16 a, columns tj + 16 b.  A step
+// passes one column and the scaled pivot row through LDS (two barriers; double
+// buffered), every wave finds the pivot by itself, and rows stay where they
+// are: with p_k the pivot row of step k, A^-1[k][p_j] is left at [p_k][j].
+// Bound by a step's latency; in LDS alone each step moved the whole block
+// three times and divided an index per entry (4096 blocks of 64 x 64: 1400 ->
+// 397 us).
+template <class T, int A>
+__global__ __launch_bounds__(256) void block_inverse_tile_kernel(int nslots, int bs, const double* __restrict__ J,
+                                                                 T* __restrict__ Dinv, int* __restrict__ nsingular,
+                                                                 int transposed) {
+    __shared__ double col[2][16 * A], row[2][16 * A];
+    __shared__ int pk[16 * A], kp[16 * A];  // pivot row of a step, step of a row
+    const int tid = threadIdx.x, ti = tid >> 4, tj = tid & 15, lane = tid & 63;
+    const double* src = J + (size_t)blockIdx.x * nslots * bs * bs;
+    T* dst = Dinv + (size_t)blockIdx.x * bs * bs;
+    double v[A][A];
+#pragma unroll
+    for (int a = 0; a < A; ++a)
+#pragma unroll
+        for (int b = 0; b < A; ++b) {
+            const int i = ti + 16 * a, c = tj + 16 * b;
+            v[a][b] = i < bs && c < bs ? src[(size_t)i * bs + c] : 0.0;
+        }
+    bool free_row = lane < bs, bad = false;  // of row `lane`
+#pragma unroll
+    for (int kb = 0; kb < A; ++kb) {
+        const int kend = min(16, bs - 16 * kb);
+        for (int kt = 0; kt < kend && !bad; ++kt) {
+            const int k = 16 * kb + kt, buf = k & 1;
+            if (tj == kt)
+#pragma unroll
+                for (int a = 0; a < A; ++a) col[buf][ti + 16 * a] = v[a][kb];
+            __syncthreads();
+            const double mine = free_row ? fabs(col[buf][lane]) : -1.0;
+            double best = mine > -1.0 ? mine : -1.0;
+            int pr = lane;
+            for (int off = 32; off > 0; off >>= 1) {
+                const double ob = __shfl_xor(best, off);
+                const int oi = __shfl_xor(pr, off);
+                if (ob > best || (ob == best && oi < pr)) {
+                    best = ob;
+                    pr = oi;
+                }
+            }
+            if (!(best > 0.0)) {
+                bad = true;  // the same in every wave
+                break;
+            }
+            if (lane == pr) free_row = false;
+            if (tid == 0) {
+                pk[k] = pr;
+                kp[pr] = k;
+            }
+            const double ipiv = 1.0 / col[buf][pr];
+#pragma unroll
+            for (int a = 0; a < A; ++a)
+                if (ti + 16 * a == pr)
+#pragma unroll
+                    for (int b = 0; b < A; ++b) {
+                        v[a][b] = (b == kb && tj == kt ? 1.0 : v[a][b]) * ipiv;
+                        row[buf][tj + 16 * b] = v[a][b];
+                    }
+            __syncthreads();
+            double rc[A];
+#pragma unroll
+            for (int b = 0; b < A; ++b) rc[b] = row[buf][tj + 16 * b];
+#pragma unroll
+            for (int a = 0; a < A; ++a) {
+                if (ti + 16 * a == pr) continue;
+                const double f = col[buf][ti + 16 * a];
+#pragma unroll
+                for (int b = 0; b < A; ++b) v[a][b] = (b == kb && tj == kt ? 0.0 : v[a][b]) - f * rc[b];
+            }
+        }
+    }
+    __syncthreads();
+    if (bad && tid == 0) atomicAdd(nsingular, 1);
+#pragma unroll
+    for (int a = 0; a < A; ++a)
+#pragma unroll
+        for (int b = 0; b < A; ++b) {
+            const int i = ti + 16 * a, c = tj + 16 * b;
+            if (i >= bs || c >= bs) continue;
+            if (bad) {
+                dst[(size_t)i * bs + c] = (T)(i == c ? 1.0 : 0.0);
+            } else {
+                const int r = kp[i], q = pk[c];
+                dst[transposed ? (size_t)q * bs + r : (size_t)r * bs + q] = (T)v[a][b];
+            }
+        }
+}
+
 // Block LU of a block-tridiagonal matrix (a chain of elements e = 0..n-1,
 // slot 1 = element e-1, slot 2 = element e+1), one wave walking the chain:
 // S_0 = D_0, S_e = D_e - L_e W_{e-1}, W_e = S_e^-1 U_e, with L_e = J[e][1],
@@ -404,7 +498,14 @@ int block_inverse(int nelem, int nslots, int bs, const double* J, T* Dinv, int* 
                   hipStream_t st) {
     const size_t sh = (size_t)bs * bs * sizeof(double) + (size_t)bs * sizeof(int);
     if (sh > 160 * 1024) return -1;
-    block_inverse_kernel<T><<<nelem, 256, sh, st>>>(nelem, nslots, bs, J, Dinv, nsingular, transposed ? 1 : 0);
+    const int tr = transposed ? 1 : 0;
+    switch ((bs + 15) / 16) {
+    case 1: block_inverse_tile_kernel<T, 1><<<nelem, 256, 0, st>>>(nslots, bs, J, Dinv, nsingular, tr); break;
+    case 2: block_inverse_tile_kernel<T, 2><<<nelem, 256, 0, st>>>(nslots, bs, J, Dinv, nsingular, tr); break;
+    case 3: block_inverse_tile_kernel<T, 3><<<nelem, 256, 0, st>>>(nslots, bs, J, Dinv, nsingular, tr); break;
+    case 4: block_inverse_tile_kernel<T, 4><<<nelem, 256, 0, st>>>(nslots, bs, J, Dinv, nsingular, tr); break;
+    default: block_inverse_kernel<T><<<nelem, 256, sh, st>>>(nelem, nslots, bs, J, Dinv, nsingular, tr);
+    }
     return (int)hipGetLastError();
 }
 template int block_inverse<float>(int, int, int, const double*, float*, int*, bool, hipStream_t);
