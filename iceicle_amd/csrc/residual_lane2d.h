@@ -8,8 +8,10 @@
 // lanes.  Operators that the lanes share are scalar loads; lines and rows meet
 // in LDS, through which the coefficients and the result also pass so that
 // memory sees whole lines.  The neighbours' coefficients are read in place.  A
-// face is a straight edge: its normal, arc length and DDG distance are read
-// once, not once a point.
+// face is a straight edge: its normal, arc length and, between two elements,
+// DDG distance n . (cR - cL) are read once, not once a point.  On a boundary
+// face the distance is sum_d |n_d (x_d - c_d)|, which varies along an edge that
+// is oblique to the axes: read at each point.
 //
 // Explicit stages (residual, inverse mass, combination) over the 96 784 to
 // 160 809 elements of a study's P1 to P3 and the 67 572 of its P4: 19 / 36 / 38
@@ -190,8 +192,9 @@ __global__ __launch_bounds__(64, lane2d_waves(P + 1)) void lane2d_kernel(DevSpac
                     const double bvp = dd.bval[(size_t)b * N + qf];
                     const VT nv[2] = {(VT)n[0], (VT)n[1]};
                     const VT uI[1] = {(VT)uO}, jd[1] = {(VT)(bvp - uO)}, bv[1] = {(VT)bvp};
+                    const VT hb = (VT)fg[qf * 4 + 3];
                     VT uB[1];
-                    boundary_point_flux<2, PH>(pf, info_bctype(rec.y), rec.z, uI, gr, bv, nv, (VT)h, (VT)ws, Q, uB, jd);
+                    boundary_point_flux<2, PH>(pf, info_bctype(rec.y), rec.z, uI, gr, bv, nv, hb, (VT)ws, Q, uB, jd);
                 }
             }
             const double qv = side ? -(double)Q[0] : (double)Q[0];
