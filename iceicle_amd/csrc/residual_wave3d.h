@@ -1,8 +1,9 @@
-// 3D residual of fluxes without a gradient (Euler) in one launch, P2 and P3,
-// without LDS: a wave owns four elements, axes 0 and 2 of their tensors lie
-// in the lanes (wave_tensor.h) and axis 1 in registers.  Contractions along
-// the lane axes are FP64 matrix instructions, along axis 1 plain FMAs, so no
-// value changes lanes otherwise.  Layouts (hi, lo): nodes (i0, i2), volume
+// 3D residual of fluxes without a gradient (Euler) in one launch, P2 and P3: a
+// wave owns four elements, axes 0 and 2 of their tensors lie in the lanes
+// (wave_tensor.h) and axis 1 in registers.  Contractions along the lane axes
+// are FP64 matrix instructions, along axis 1 plain FMAs; the own nodes of a
+// face of axis 0 or 2 come from other lanes through the wave's part of LDS
+// (51 KB a workgroup at P3, no barriers).  Layouts (hi, lo): nodes (i0, i2), volume
 // points (q2, q0), points of the faces of axis 0 (q2, q1), axis 1 (q2, q0),
 // axis 2 (q0, q1).
 //
@@ -213,6 +214,10 @@ __global__ __launch_bounds__(256, ICE_WAVE3D_MINW) void wave3d_kernel(DevSpace S
     }
 
     // ---- faces
+    // (the faces read coefficients that other lanes of the wave stashed)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     double lt[N];  // L0[point hi][node i]: the lifting operators along axis 1
 #pragma unroll
     for (int i = 0; i < N; ++i) lt[i] = kin ? L0[hc * N + i] : 0.0;
