@@ -2180,6 +2180,19 @@ int profiled(hipEvent_t* ev, hipStream_t st, F launch) {
     return rc;
 }
 
+// The state a one-launch residual reads when R is to replace U: its waves read
+// the coefficients of elements whose residual other waves store, so a copy, in
+// the trace buffer of the three launches (4 N or more values an element and
+// variable in 2D, 6 N^2 in 3D, to the coefficients' N^D <= 5 N, 4 N^2).
+int separate_state(const DevSpace& S, int flux, const DiscDev& dd, const double* R, hipStream_t st, const double** U) {
+    if (*U != R) return 0;
+    size_t n = (size_t)S.nelem * (flux == ICE_FLUX_BURGERS ? 1 : S.ndim + 2);
+    for (int d = 0; d < S.ndim; ++d) n *= S.n;
+    const int rc = (int)hipMemcpyAsync(dd.T, R, n * sizeof(double), hipMemcpyDeviceToDevice, st);
+    *U = dd.T;
+    return rc;
+}
+
 int residual_stage(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                    const double* U, double* K, const StageComb<double>& cb, hipStream_t st) {
     if (!wave_covers(ndim, p, flux, dd)) return -2;
@@ -2213,7 +2226,8 @@ int residual_fp64(int ndim, int p, int flux, const DevSpace& S, const PhysParams
                   const double* U, double* R, hipStream_t st, hipEvent_t* ev) {
     if (wave_covers(ndim, p, flux, dd))
         return profiled(ev, st, [&] {
-            return wave_residual<double>(flux, p, S, ph, dd, U, R, (double*)nullptr, StageComb<double>{}, st);
+            const int rc = separate_state(S, flux, dd, R, st, &U);
+            return rc ? rc : wave_residual<double>(flux, p, S, ph, dd, U, R, (double*)nullptr, StageComb<double>{}, st);
         });
     if (flux == ICE_FLUX_BURGERS) {
         if (ndim == 1) return dispatch_order<Burgers<1>, 1>(p, S, ph, dd, U, R, st, ev);
@@ -2247,7 +2261,10 @@ int residual_mixed_dim(int p, int flux, const DevSpace& S, const PhysParams& ph,
 int residual_mixed(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                    const double* U, double* R, hipStream_t st, hipEvent_t* ev) {
     if (wave_covers(ndim, p, flux, dd))
-        return profiled(ev, st, [&] { return wave_residual<float>(flux, p, S, phys_cast<float>(ph), dd, U, R, st); });
+        return profiled(ev, st, [&] {
+            const int rc = separate_state(S, flux, dd, R, st, &U);
+            return rc ? rc : wave_residual<float>(flux, p, S, phys_cast<float>(ph), dd, U, R, st);
+        });
     if (ndim == 2) return residual_mixed_dim<2, double>(p, flux, S, ph, dd, U, R, st, ev);
     if (ndim == 3) return residual_mixed_dim<3, double>(p, flux, S, ph, dd, U, R, st, ev);
     return -2;

@@ -311,7 +311,8 @@ def form_residual(space, disc, u, res, stream=None, precision="fp64"):
     or "mixed" (FP32 fluxes, FP64 geometry and output, 2D and 3D).
     u may be an FP32 state (2D and 3D): "mixed" is then the residual FP32
     steps use, "fp64" the FP64 residual of the widened state (the check of an
-    FP32 solution against the FP64 discretization).  res is float64."""
+    FP32 solution against the FP64 discretization).  res is float64; it may be
+    u itself but not overlap it in any other way."""
     import torch
     _require_cuda(res, "res")
     if isinstance(u, torch.Tensor) and u.dtype == torch.float32:

@@ -271,7 +271,9 @@ int ice_disc_autotune(ice_disc* disc, const double* u_dev, double* r_dev, int re
                       void* stream);
 
 /* form_residual (form_residual.hpp:56-268): res <- R(u), FP64, device pointers
- * in fe_layout_right order, both nelem*nbasis*neq doubles. */
+ * in fe_layout_right order, both nelem*nbasis*neq doubles.  res may be u
+ * itself (also in the mixed-precision and allocation-free forms below); the
+ * two may not overlap in any other way. */
 int ice_residual(ice_disc* disc, const double* u_dev, double* res_dev, void* stream);
 
 /* Mixed-precision residual (no reference counterpart; the reference is FP64

@@ -211,3 +211,26 @@ def test_mixed_ns_mms_128_p3_against_fp64():
         err = float((r32 - r64).abs().max() / r64.abs().max())
         print(f"NS MMS 128x128 P3 {name}: mixed vs fp64 rel err {err:.3e}", flush=True)
         assert err <= tol
+
+
+@pytest.mark.parametrize("ndim,order,flux", [(1, 3, abi.FLUX_BURGERS), (2, 2, abi.FLUX_BURGERS), (2, 4, abi.FLUX_BURGERS),
+                                             (2, 3, abi.FLUX_NAVIER_STOKES), (2, 4, abi.FLUX_NAVIER_STOKES),
+                                             (2, 1, abi.FLUX_EULER), (3, 3, abi.FLUX_EULER), (3, 1, abi.FLUX_EULER)])
+def test_residual_in_place(ndim, order, flux):
+    """R(u) may replace u: the same bits as in a buffer of its own."""
+    from iceicle_amd import engine
+    nel = [40, 33, 12][:ndim]
+    m = abi.mesh_desc(ndim, nel, [0.0] * ndim, [1.0] * ndim, ["DIRICHLET"] * (2 * ndim))
+    p = cases.burgers_params(ndim) if flux == abi.FLUX_BURGERS else cases.ns_params(ndim, flux=flux)
+    space = engine.FESpace(m, order)
+    disc = engine.ConservationLawDDG(space, p)
+    u = torch.from_numpy(cases.random_state(flux, ndim, space.nelem, space.nbasis, 3)).cuda()
+    calls = [lambda x, r: engine.form_residual(space, disc, x, r)]
+    if ndim > 1:
+        calls.append(lambda x, r: engine.form_residual(space, disc, x, r, precision="mixed"))
+    for call in calls:
+        r, w = torch.empty_like(u), u.clone()
+        call(u, r)
+        call(w, w)
+        torch.cuda.synchronize()
+        assert torch.equal(w, r)
