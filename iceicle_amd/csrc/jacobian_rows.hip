@@ -35,6 +35,12 @@ typedef double doublex4 __attribute__((ext_vector_type(4)));
 
 constexpr double SQRT_EPS = 1.4901161193847656e-08;  // sqrt(DBL_EPSILON)
 
+// Step of the gradient arguments.  The flux is linear in them, so a step has
+// no truncation error whatever its size, and a large one leaves the total
+// flux's rounding behind: with a unit step in SI units (air, energy flux 4e7,
+// viscosity 1.8e-5) entries that are viscous only were up to 2e-4 off.
+constexpr double GRAD_STEP = 0x1p40, INV_GRAD_STEP = 0x1p-40;
+
 template <int D, int P, class PH>
 struct RowShape {
     static constexpr int N = P + 1, NB = Pow<N, D>::value, NFQ = Pow<N, D - 1>::value, M = PH::M, NBM = NB * M;
@@ -350,17 +356,17 @@ __global__ __launch_bounds__((RowShape<D, P, PH>::THREADS), 2) void jac_row_kern
 #pragma unroll
                 for (int v = 0; v < M; ++v) dA[k / M][p][v][w] = (Q[v] - fQ[p][v]) * ieps;
             } else {
-                // linear in the gradient: its unit step is exact to rounding
+                // linear in the gradient: exact to rounding
 #pragma unroll
                 for (int v = 0; v < M; ++v) {
                     uO[v] = fu[0][p][v];
                     uN[v] = fu[1][p][v];
                 }
 #pragma unroll
-                for (int i = 0; i < MD; ++i) g[i] = fg[p][i] + (k - 2 * M == i ? 1.0 : 0.0);
+                for (int i = 0; i < MD; ++i) g[i] = fg[p][i] + (k - 2 * M == i ? GRAD_STEP : 0.0);
                 face_flux(p, uO, uN, g, Q);
 #pragma unroll
-                for (int v = 0; v < M; ++v) dB[p][v][k - 2 * M] = Q[v] - fQ[p][v];
+                for (int v = 0; v < M; ++v) dB[p][v][k - 2 * M] = (Q[v] - fQ[p][v]) * INV_GRAD_STEP;
             }
         } else {
             const int s = t - FP * NPF, q = s / NPV, k = s % NPV;
@@ -369,7 +375,7 @@ __global__ __launch_bounds__((RowShape<D, P, PH>::THREADS), 2) void jac_row_kern
 #pragma unroll
             for (int v = 0; v < M; ++v) u[v] = vu[q][v] + (k == v ? eps : 0.0);
 #pragma unroll
-            for (int i = 0; i < MD; ++i) g[i] = vgr[q][i] + (k - M == i ? 1.0 : 0.0);
+            for (int i = 0; i < MD; ++i) g[i] = vgr[q][i] + (k - M == i ? GRAD_STEP : 0.0);
             PH::flux(ph, u, g, F);
 #pragma unroll
             for (int v = 0; v < M; ++v)
@@ -377,7 +383,7 @@ __global__ __launch_bounds__((RowShape<D, P, PH>::THREADS), 2) void jac_row_kern
                 for (int d = 0; d < D; ++d) {
                     const double df = F[v * D + d] - vF[q][v * D + d];
                     if (k < M) dFu[q][v][d][k] = df * ieps;
-                    else dFg[q][v][d][k - M] = df;
+                    else dFg[q][v][d][k - M] = df * INV_GRAD_STEP;
                 }
         }
     }
