@@ -19,6 +19,7 @@ struct MGCells {
     int coff[MG_MAX_COLOURS + 1];
     const int* children;  // [n][8] cells of the finer level
     const int* parent;    // [n] cell of the coarser level
+    bool settled;         // a symmetric sweep leaves colour 0 no residual (no cell is its own neighbour)
 };
 
 // The levels one workgroup takes through a V-cycle
@@ -46,8 +47,9 @@ int mg_prolong_residual(int nslots, int m, const MGCells& L, const double* b, co
                         double* r, hipStream_t st);
 // x += P xc + t
 int mg_prolong_add(int m, const MGCells& L, const double* xc, const double* t, double* x, hipStream_t st);
-// fine level: r = v - J x of a completed sweep (zero on colour 0) and its
-// element sums b0; then out += P x0, r -= (J P) x0
+// fine level: r = v - J x of a completed sweep that leaves colour 0 no residual
+// (it is not formed there) and its element sums b0; then out += P x0,
+// r -= (J P) x0
 template <class T>
 int mg_fine_residual(int nelem, int nslots, int bs, int m, const int* cols, const int* ecolor, const T* JT,
                      const double* x, const double* v, double* r, double* b0, hipStream_t st);

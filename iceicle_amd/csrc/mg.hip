@@ -10,7 +10,9 @@
 //  - The levels that fit one workgroup's LDS (up to about 1300 cells in all
 //    at m = 4) run to the bottom and back in one launch, vectors in LDS.
 //  - After a symmetric sweep the rows of colour 0, solved last, have no
-//    residual; on the fine level that halves the residual, and after the
+//    residual (unless a cell is its own neighbour, in a periodic direction of
+//    one cell: the sweep leaves that coupling out, and the residual is formed
+//    on every row); on the fine level that halves the residual, and after the
 //    coarse correction x += P xc the residual is updated with the precomputed
 //    J P (a sixteenth of the bytes at 16 nodes an element) instead of formed again.
 // 2D NS P3 64 x 64, an iteration of GMRES with its operator: 710 -> 460 us
@@ -122,7 +124,7 @@ __global__ __launch_bounds__(256) void residual_restrict_kernel(MGCells L, MGCel
     double s = 0.0;
     for (int k = 0; k < 8; ++k) {
         const int e = C.children[(size_t)P * 8 + k];
-        if (e < 0 || before(L, e, 1)) continue;
+        if (e < 0 || (L.settled && before(L, e, 1))) continue;
         s += b[(size_t)e * M + r] - row_sum<M, NS>(
                                         L, e, r, [](int, int) { return true; },
                                         [&](int col, int c) { return x[(size_t)col * M + c]; });
@@ -208,7 +210,7 @@ __global__ __launch_bounds__(TAIL_THREADS) void tail_kernel(MGTail T, const doub
         const MGCells& C = T.lev[l + 1];
         double *b = x + L.n * M, *t = b + L.n * M, *xn = t + L.n * M;
         sweep(L, b, x);
-        residual(L, b, x, t, true);
+        residual(L, b, x, t, L.settled);
         for (int i = tid; i < C.n * M; i += TAIL_THREADS) {
             const int P = i / M, v = i - P * M;
             double s = 0.0;

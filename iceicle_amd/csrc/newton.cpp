@@ -98,6 +98,7 @@ struct MGLevel {
     int n = 0;
     int dims[3] = {1, 1, 1};
     std::vector<int> hcols;        // [n][nslots]
+    bool settled = true;           // MGCells
     std::vector<int> at;           // [n] lexicographic grid position (level 0: the cell number)
     const int* cols = nullptr;     // device copy of hcols
     int* parent = nullptr;         // [n] cell of the next coarser level (null on the coarsest)
@@ -281,6 +282,7 @@ struct ice_newton {
         for (int k = 0; k <= c.ncol; ++k) c.coff[k] = L.coff[k];
         c.children = L.children;
         c.parent = L.parent;
+        c.settled = L.settled;
         return c;
     }
 
@@ -326,6 +328,9 @@ struct ice_newton {
         int ns = 0, b = 0;
         if (ice_jacobian_layout(disc, &ns, &b, L0.hcols.data()) != ICE_OK) throw Fail{ICE_ERR_STATE, "no layout"};
         L0.cols = ice::disc_jcols(disc);
+        // (on the coarser levels such couplings are part of the diagonal)
+        for (size_t k = 0; k < L0.hcols.size(); ++k)
+            if (k % nslots && L0.hcols[k] == (int)(k / nslots)) L0.settled = false;
         mg.push_back(std::move(L0));
         while (mg.back().n > 64 && mg.size() < 16) {
             MGLevel& F = mg.back();
@@ -401,7 +406,7 @@ struct ice_newton {
         tail.nlev = (int)mg.size() - tail_level;
         for (int l = 0; l < tail.nlev; ++l) tail.lev[l] = cells(tail_level + l);
         fine_ap = alloc<float>((size_t)nelem * nslots * bs * neq);
-        fine_fused = ice::mg_fine_covers(bs, neq, J16 ? 2 : 4);
+        fine_fused = mg[0].settled && ice::mg_fine_covers(bs, neq, J16 ? 2 : 4);
         coarse_n = mg.back().n * neq;
         if (coarse_n <= 1024) coarse_inv = alloc<double>((size_t)coarse_n * coarse_n);
     }

@@ -63,3 +63,36 @@ def test_multigrid_linear_solve(flux, order, nel, bc, smoother, rate):
         assert abs(true - rel) <= 1e-3 * rel + 1e-14
     assert abs(got[abi.PC_MULTIGRID] - rate) <= 2e-3
     assert got[abi.PC_MULTIGRID] < got[abi.PC_BLOCK_SGS]
+
+
+@pytest.mark.parametrize("flux,order,nel", [("burgers", 1, [300, 1]), ("burgers", 2, [300, 1]), ("burgers", 3, [256, 1]),
+                                            ("ns", 1, [100, 1]), ("ns", 3, [64, 1]), ("burgers", 1, [300, 1, 1])])
+def test_periodic_directions_of_one_element(flux, order, nel):
+    """Elements that are their own neighbours, three times as narrow there as
+    long: after 60 iterations the cycle's residual is below a fifteenth of the
+    smoother's (measured 1/2300 to 1/114 with the residual of the sweep formed on
+    every row; taken for zero on colour 0, 1/4 to 2.3 times the
+    smoother's)."""
+    from iceicle_amd import engine
+    dim = len(nel)
+    bc = ([D] + [P] * (dim - 1)) * 2
+    m = abi.mesh_desc(dim, nel, [0.0] * dim, [float(nel[0])] + [1.0 / 3.0] * (dim - 1), bc,
+                      periodic_mode=abi.PERIODIC_COUPLED)
+    if flux == "burgers":
+        p = cases.burgers_params(dim, mu=5.0, a=(0.3, -0.2, 0.1), b=(0.2, 0.1, -0.1))
+    else:
+        p = cases.ns_params(dim, mu=0.5)
+    disc = engine.ConservationLawDDG(engine.FESpace(m, order), p)
+    rng = np.random.default_rng(7)
+    nv = 1 if flux == "burgers" else dim + 2
+    base = [0.2] if nv == 1 else [1.0, 0.3] + [0.0] * (dim - 1) + [1.0 / 1.4 / 0.4 + 0.045]
+    u = torch.from_numpy(np.tile(base, disc.size // nv) + 1e-3 * rng.uniform(-1, 1, disc.size)).cuda()
+    b = torch.from_numpy(rng.normal(size=disc.size)).cuda()
+    got = {}
+    for pc in (abi.PC_MULTIGRID, abi.PC_BLOCK_SGS):
+        solver = engine.PetscNewton(disc, linear_rtol=1e-12, gmres_maxit=60, gmres_restart=60, preconditioner=pc)
+        x = torch.full_like(u, float("nan"))
+        got[pc] = solver.linear_solve(b, x, u=u)[1]
+    ratio = got[abi.PC_MULTIGRID] / got[abi.PC_BLOCK_SGS]
+    print(flux, order, nel, f"{ratio:.2e}", flush=True)
+    assert ratio <= 1 / 15
