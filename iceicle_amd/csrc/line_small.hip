@@ -270,6 +270,7 @@ __global__ __launch_bounds__(PCR_THREADS) void pcr_factor_kernel(int n, int nslo
                                                                  double* work, int* nsingular) {
     constexpr int BB = BS * BS;
     __shared__ int chain;
+    __shared__ double size[PCR_MAX_ROWS];  // largest entry a row's diagonal block had or lost (the row's thread's own)
     const size_t blk = (size_t)BB * n;
     double *I = work + PCR_HEAD, *cur = I + blk, *nxt = cur + 3 * blk, *AC = nxt + 3 * blk;
     const int tid = threadIdx.x;
@@ -282,6 +283,7 @@ __global__ __launch_bounds__(PCR_THREADS) void pcr_factor_kernel(int n, int nslo
             cur[blk + (size_t)k * n + e] = e > 0 ? Je[BB + k] : 0.0;
             cur[2 * blk + (size_t)k * n + e] = e + 1 < n ? Je[2 * BB + k] : 0.0;
         }
+        size[e] = 0.0;
     }
     __syncthreads();
     for (int s = 1;; s <<= 1) {
@@ -289,7 +291,8 @@ __global__ __launch_bounds__(PCR_THREADS) void pcr_factor_kernel(int n, int nslo
             double M[BB], Inv[BB];
             get<BS>(cur, n, e, M);
             const bool ok = small_inverse<BS>(M, Inv);
-            if (!ok || !(largest<BS>(M) * largest<BS>(Inv) <= 1e10)) chain = 1;
+            size[e] = fmax(size[e], largest<BS>(M));
+            if (!ok || !(size[e] * largest<BS>(Inv) <= 1e10)) chain = 1;
             put<BS>(s < n ? I : Sinv, n, e, Inv);
         }
         __syncthreads();
@@ -307,6 +310,7 @@ __global__ __launch_bounds__(PCR_THREADS) void pcr_factor_kernel(int n, int nslo
                 mul<BS>(A, X, T);
 #pragma unroll
                 for (int k = 0; k < BB; ++k) nD[k] -= T[k];
+                size[e] = fmax(size[e], largest<BS>(T));
                 get<BS>(cur + off * blk, n, f, X);
                 mul<BS>(A, X, T);
 #pragma unroll
