@@ -5,6 +5,7 @@
 namespace ice {
 
 constexpr int MG_MAX_LEVELS = 16, MG_MAX_COLOURS = 8;
+constexpr int MG_DIRECT = 1024;  // unknowns of a last level solved exactly, at most: one a thread of the tail
 
 // n cells with m x m blocks in the Jacobian's slots (slot 0 the cell itself),
 // blocks and factored diagonals FP32 with the cells' rows contiguous, so that
@@ -26,7 +27,7 @@ struct MGCells {
 struct MGTail {
     int nlev;
     MGCells lev[MG_MAX_LEVELS];
-    const double* inv;    // dense inverse of the last level (column-major), or null
+    const double* inv;    // dense inverse of the last level (column-major, up to MG_DIRECT unknowns), or null
 };
 
 // the blocks' FP32 copies in that layout, from row-major FP64 blocks and

@@ -166,7 +166,7 @@ __global__ void pack_kernel(int n, int nslots, int m, const double* __restrict__
     }
 }
 
-constexpr int TAIL_THREADS = 1024;
+constexpr int TAIL_THREADS = MG_DIRECT;
 
 // The V-cycle of T's levels in one workgroup, three vectors a level in LDS:
 // solution, right-hand side (later the correction), residual.
@@ -231,24 +231,16 @@ __global__ __launch_bounds__(TAIL_THREADS) void tail_kernel(MGTail T, const doub
             // rows in the threads' low part, columns split over the rest
             const int nr = (n + 63) & ~63, np = TAIL_THREADS / nr, i = tid % nr, p = tid / nr;
             double s = 0.0;
-            if (np > 0) {
-                if (p < np && i < n) {
+            if (p < np && i < n) {
 #pragma unroll 16
-                    for (int j = p; j < n; j += np) s += T.inv[(size_t)j * n + i] * b[j];
-                }
-                part[tid] = s;
-                __syncthreads();
-                if (tid < n) {
-                    s = 0.0;
-                    for (int k = 0; k < np; ++k) s += part[k * nr + tid];
-                    x[tid] = s;
-                }
-            } else {
-                for (int k = tid; k < n; k += TAIL_THREADS) {
-                    s = 0.0;
-                    for (int j = 0; j < n; ++j) s += T.inv[(size_t)j * n + k] * b[j];
-                    x[k] = s;
-                }
+                for (int j = p; j < n; j += np) s += T.inv[(size_t)j * n + i] * b[j];
+            }
+            part[tid] = s;
+            __syncthreads();
+            if (tid < n) {
+                s = 0.0;
+                for (int k = 0; k < np; ++k) s += part[k * nr + tid];
+                x[tid] = s;
             }
             __syncthreads();
         } else {

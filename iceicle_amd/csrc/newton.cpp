@@ -408,11 +408,11 @@ struct ice_newton {
         fine_ap = alloc<float>((size_t)nelem * nslots * bs * neq);
         fine_fused = mg[0].settled && ice::mg_fine_covers(bs, neq, J16 ? 2 : 4);
         coarse_n = mg.back().n * neq;
-        if (coarse_n <= 1024) coarse_inv = alloc<double>((size_t)coarse_n * coarse_n);
+        if (coarse_n <= ice::MG_DIRECT) coarse_inv = alloc<double>((size_t)coarse_n * coarse_n);
     }
 
     // dense inverse of the coarsest level by Gauss-Jordan with partial
-    // pivoting on the host (at most 1024 unknowns), uploaded column-major;
+    // pivoting on the host (at most MG_DIRECT unknowns), uploaded column-major;
     // false if the level is singular (the V-cycle then keeps its SGS sweeps)
     bool factor_coarse(hipStream_t st) {
         if (!coarse_inv) return false;
