@@ -876,10 +876,12 @@ int ice_disc_autotune(ice_disc* d, const double* u, double* r, int reps, int* be
     int pick = 0, pick_mixed = 0;
     int rc = ICE_OK;
     // FP64 residual, then the mixed one (its own tile: FP32 tiles hold half
-    // the bytes, so the fastest shape can differ)
+    // the bytes, so the fastest shape can differ); the one-launch kernels have
+    // one shape, timed as tile 0 and reported for all
+    const int ntile = ice::wave_covers(s->ndim, s->p, d->prm.flux, d->dd) ? 1 : 3;
     for (int prec = 0; prec < 2 && rc == ICE_OK; ++prec) {
         double tbest = 1e300;
-        for (int tile = 0; tile < 3 && rc == ICE_OK; ++tile) {
+        for (int tile = 0; tile < ntile && rc == ICE_OK; ++tile) {
             d->dd.tile = tile;
             d->dd.tile_mixed = tile;
             auto once = [&]() {
@@ -900,7 +902,8 @@ int ice_disc_autotune(ice_disc* d, const double* u, double* r, int reps, int* be
                 break;
             }
             const double per = (double)t / reps;
-            if (ms && prec == 0) ms[tile] = per;
+            if (ms && prec == 0)
+                for (int t = tile; t < (ntile == 1 ? 3 : tile + 1); ++t) ms[t] = per;
             if (per < tbest) {
                 tbest = per;
                 (prec == 0 ? pick : pick_mixed) = tile;

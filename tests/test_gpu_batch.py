@@ -148,3 +148,17 @@ def test_full_batch_of_512_instances():
     for g, m0 in zip(bt.groups, umax0):
         assert bool(torch.isfinite(g.u).all()), g.order
         assert float(g.u.abs().max()) <= 1.05 * m0, (g.order, float(g.u.abs().max()), m0)
+
+
+@pytest.mark.parametrize("order,one_launch", [(2, True), (4, False)])
+def test_autotune_of_one_shape(order, one_launch):
+    """A residual of one launch has one shape: tile 0 and one time, reported
+    for all three; the three launches (Euler P4) are timed one tile at a time."""
+    from iceicle_amd import engine
+    m = abi.mesh_desc(2, [9, 8], [0.0, 0.0], [1.0, 1.0], ["EXTRAPOLATION"] * 4)
+    disc = engine.ConservationLawDDG(engine.FESpace(m, order), abi.default_params(abi.FLUX_EULER))
+    u = torch.from_numpy(np.tile([1.0, 0.3, 0.1, 2.0], disc.size // 4)).cuda()
+    best, ms = disc.autotune(u, torch.empty_like(u), reps=3)
+    assert all(t > 0.0 for t in ms) and best in (0, 1, 2)
+    if one_launch:
+        assert best == 0 and len(set(ms)) == 1
