@@ -1,5 +1,7 @@
 """Batched instances: a batched space evaluates every instance exactly as
-its own space does (bit for bit), per-element viscosities and step sizes
+its own space does (bit for bit where both take the same kernel, as here: see
+test_gpu_lane2d for a space of elements enough for the lanes against one that
+has not), per-element viscosities and step sizes
 reproduce per-instance runs, HIP-graph replay reproduces eager stepping,
 and every element-kernel tile gives the same residual."""
 import numpy as np
