@@ -145,3 +145,28 @@ def test_cfl_step_graph_matches_eager():
     g.launch()
     torch.cuda.synchronize()
     assert torch.equal(keep, ub)
+
+
+@pytest.mark.parametrize("flux,nel", [(abi.FLUX_NAVIER_STOKES, [64, 64]), (abi.FLUX_NAVIER_STOKES, [67, 62]),
+                                      (abi.FLUX_EULER, [127, 129]), (abi.FLUX_NAVIER_STOKES, [131, 129]),
+                                      (abi.FLUX_BURGERS, [61, 65]), (abi.FLUX_BURGERS, [257, 257])])
+def test_cfl_steps_of_many_waves(flux, nel):
+    """Wave speeds of four elements a wave (Burgers lanes: 16) folded by one
+    small, one large and several workgroups (1024 and 4096 waves, and a few on
+    either side): the step sizes of the oracle to rounding, the fastest state
+    in one corner element."""
+    from iceicle_amd import engine
+    m = abi.mesh_desc(2, nel, [0, 0], [1, 1], ["EXTRAPOLATION"] * 4)
+    prm = abi.default_params(flux)
+    prm.visc_mu = prm.mu = 0.01
+    o, space, disc = _setup(m, 1, prm)
+    for corner in (0, o.nelem - 1):
+        u0 = np.tile([0.3] if flux == abi.FLUX_BURGERS else [1.0, 0.3, 0.1, 2.0], (o.nelem, 4, 1))
+        u0[corner, :, -1] *= 2.0
+        u0 = u0.ravel()
+        ref, n_ref, t_ref = o.rk_solve(u0, kind=0, cfl=0.3, ntime=3)
+        u = torch.from_numpy(u0).cuda()
+        n, t = engine.ExplicitStepper(disc, abi.stepper_desc(abi.STEP_RK3_SSP, cfl=0.3, ntime=3)).solve(u)
+        err = cases.rel_inf(u.cpu().numpy(), ref)
+        print(f"{nel} corner {corner}: t {t:.6e} ({t_ref:.6e}) err {err:.1e}", flush=True)
+        assert n == n_ref == 3 and abs(t - t_ref) <= 1e-13 * t_ref and err <= 1e-12
