@@ -878,7 +878,7 @@ int ice_disc_autotune(ice_disc* d, const double* u, double* r, int reps, int* be
     // FP64 residual, then the mixed one (its own tile: FP32 tiles hold half
     // the bytes, so the fastest shape can differ); the one-launch kernels have
     // one shape, timed as tile 0 and reported for all
-    const int ntile = ice::wave_covers(s->ndim, s->p, d->prm.flux, d->dd) ? 1 : 3;
+    const int ntile = ice::wave_covers(s->ndim, s->p, d->prm.flux, s->mesh.nelem, d->dd) ? 1 : 3;
     for (int prec = 0; prec < 2 && rc == ICE_OK; ++prec) {
         double tbest = 1e300;
         for (int tile = 0; tile < ntile && rc == ICE_OK; ++tile) {
@@ -1241,7 +1241,7 @@ int step_once(ice_stepper* S, double* u, hipStream_t st) {
             axpy(1.0 / 6.0, k1, u);
             axpy(1.0 / 6.0, k1, u);
             axpy(2.0 / 3.0, k1, u);
-        } else if (ice::wave_covers(sp->ndim, sp->p, d->prm.flux, d->dd)) {
+        } else if (ice::stage_covers(sp->ndim, sp->p, d->prm.flux, sp->mesh.nelem, d->dd, false)) {
             // a launch per stage: residual, inverse mass and combination in
             // its increment-free form; no stage may write the state it reads
             auto stage = [&](const double* x, double cx, double* out) {
@@ -1320,7 +1320,8 @@ int step_once(ice_stepper* S, float* u, hipStream_t st) {
     };
     const float* kk[2] = {k1, k2};
     rc |= ice::launch_step_begin(S->st, d->d_wave, S->ctl, st);
-    if (S->desc.kind == ICE_STEP_RK3_SSP && ice::wave_covers(sp->ndim, sp->p, d->prm.flux, d->dd)) {
+    if (S->desc.kind == ICE_STEP_RK3_SSP &&
+        ice::stage_covers(sp->ndim, sp->p, d->prm.flux, sp->mesh.nelem, d->dd, true)) {
         auto stage = [&](const float* x, float* k, int nprev, const double* c, float* out, bool store_k) {
             const auto cb = ice::make_stage<float>(u, nprev, kk, c, dt, S->dte, S->st, out, store_k);
             rc |= ice::residual_stage(sp->ndim, sp->p, d->prm.flux, sp->dev, d->ph, d->dd, x, k, cb, st);

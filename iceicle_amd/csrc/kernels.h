@@ -123,10 +123,21 @@ int launch_step_end(StepState* s, hipStream_t st);
 
 // One-launch residuals without DDGIC vectors (residual_wave2d.h,
 // residual_lane2d.h, residual_wave3d.h): 2D P1-P3, scalar 2D P4, 3D Euler P2
-// and P3.
-inline bool wave_covers(int ndim, int p, int flux, const DiscDev& dd) {
+// and P3.  Not 2D Navier-Stokes P1 on many elements: the matrix tiles hold 4 of
+// its 16 entries, and each element costs what a P3 one does; three launches are
+// faster from about 190 x 190 (192^2 38 us for 39, 224^2 51 for 47, 320^2 95 for
+// 77; mixed 32 for 33, 43 for 37, 80 for 61).
+inline bool wave_covers(int ndim, int p, int flux, int nelem, const DiscDev& dd) {
+    if (ndim == 2 && flux == ICE_FLUX_NAVIER_STOKES && p == 1 && nelem > 36000) return false;
     return (ndim == 2 && (p <= 3 || flux == ICE_FLUX_BURGERS) && !dd.Pic) ||
            (ndim == 3 && flux == ICE_FLUX_EULER && (p == 2 || p == 3));
+}
+// Explicit stages in the launch of their residual.  Not FP64 2D Navier-Stokes P1
+// from about 155 x 155 elements, whose stages spill more than its residual (144^2
+// step 99 to 106 us for 105, 160^2 111 to 117 for 108).
+inline bool stage_covers(int ndim, int p, int flux, int nelem, const DiscDev& dd, bool fp32) {
+    if (ndim == 2 && flux == ICE_FLUX_NAVIER_STOKES && p == 1 && !fp32 && nelem > 24000) return false;
+    return wave_covers(ndim, p, flux, nelem, dd);
 }
 // The scalar 2D ones by lanes, from the element count where a step of 3
 // stages is faster than with matrix instructions, a wave of which is 4

@@ -2206,36 +2206,36 @@ int separate_state(const DevSpace& S, int flux, const DiscDev& dd, const double*
 
 int residual_stage(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                    const double* U, double* K, const StageComb<double>& cb, hipStream_t st) {
-    if (!wave_covers(ndim, p, flux, dd)) return -2;
+    if (!wave_covers(ndim, p, flux, S.nelem, dd)) return -2;
     return wave_residual<double>(flux, p, S, ph, dd, U, (double*)nullptr, K, cb, st);
 }
 
 int residual_stage(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                    const float* U, float* K, const StageComb<float>& cb, hipStream_t st) {
-    if (!wave_covers(ndim, p, flux, dd)) return -2;
+    if (!wave_covers(ndim, p, flux, S.nelem, dd)) return -2;
     return wave_residual<float>(flux, p, S, phys_cast<float>(ph), dd, U, (double*)nullptr, K, cb, st);
 }
 
 template <class PH, int D, class UT = double>
 int dispatch_order(int p, const DevSpace& S, const typename PH::Params& ph, const DiscDev& dd, const UT* U,
                    double* R, hipStream_t st, hipEvent_t* ev) {
-    // P1-P3 in 2D and the scalar P4 come here with the DDGIC lifting vectors only, 3D fluxes
-    // without a gradient not with P2 and P3 (wave_covers)
-    constexpr bool EULER3 = D == 3 && !TraceRec<PH, D>::NEED_GRAD;
+    // P1-P3 in 2D and the scalar P4 come here with the DDGIC lifting vectors only, but for
+    // large P1 with a gradient; 3D fluxes without one not with P2 and P3 (wave_covers)
+    constexpr bool GRAD = TraceRec<PH, D>::NEED_GRAD;
     if (p == 4) return launch_residual<D, 4, PH, UT>(S, ph, dd, U, R, st, ev);
-    if constexpr (D != 2 || PH::HAS_HOMOGENEITY) {
+    if constexpr (D != 2 || GRAD) {
         if (p == 1) return launch_residual<D, 1, PH, UT>(S, ph, dd, U, R, st, ev);
-        if constexpr (!EULER3) {
-            if (p == 2) return launch_residual<D, 2, PH, UT>(S, ph, dd, U, R, st, ev);
-            if (p == 3) return launch_residual<D, 3, PH, UT>(S, ph, dd, U, R, st, ev);
-        }
+    }
+    if constexpr (D == 1 || PH::HAS_HOMOGENEITY || (D == 3 && GRAD)) {
+        if (p == 2) return launch_residual<D, 2, PH, UT>(S, ph, dd, U, R, st, ev);
+        if (p == 3) return launch_residual<D, 3, PH, UT>(S, ph, dd, U, R, st, ev);
     }
     return -1;
 }
 
 int residual_fp64(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                   const double* U, double* R, hipStream_t st, hipEvent_t* ev) {
-    if (wave_covers(ndim, p, flux, dd))
+    if (wave_covers(ndim, p, flux, S.nelem, dd))
         return profiled(ev, st, [&] {
             const int rc = separate_state(S, flux, dd, R, st, &U);
             return rc ? rc : wave_residual<double>(flux, p, S, ph, dd, U, R, (double*)nullptr, StageComb<double>{}, st);
@@ -2271,7 +2271,7 @@ int residual_mixed_dim(int p, int flux, const DevSpace& S, const PhysParams& ph,
 
 int residual_mixed(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                    const double* U, double* R, hipStream_t st, hipEvent_t* ev) {
-    if (wave_covers(ndim, p, flux, dd))
+    if (wave_covers(ndim, p, flux, S.nelem, dd))
         return profiled(ev, st, [&] {
             const int rc = separate_state(S, flux, dd, R, st, &U);
             return rc ? rc : wave_residual<float>(flux, p, S, phys_cast<float>(ph), dd, U, R, st);
@@ -2285,7 +2285,7 @@ int residual_mixed(int ndim, int p, int flux, const DevSpace& S, const PhysParam
 // coefficients; differences and element values still formed in FP64)
 int residual_mixed_f32state(int ndim, int p, int flux, const DevSpace& S, const PhysParams& ph, const DiscDev& dd,
                             const float* U, double* R, hipStream_t st) {
-    if (wave_covers(ndim, p, flux, dd))
+    if (wave_covers(ndim, p, flux, S.nelem, dd))
         return wave_residual<float>(flux, p, S, phys_cast<float>(ph), dd, U, R, (float*)nullptr, StageComb<float>{}, st);
     if (ndim == 2) return residual_mixed_dim<2, float>(p, flux, S, ph, dd, U, R, st, nullptr);
     if (ndim == 3) return residual_mixed_dim<3, float>(p, flux, S, ph, dd, U, R, st, nullptr);

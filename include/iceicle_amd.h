@@ -258,7 +258,8 @@ int ice_disc_set_element_viscosity(ice_disc* disc, const double* mu);
  * number of variables and dimension are fixed): tile 0 = whole elements in
  * 256 threads (default), 1 = 128, 2 = 64, 3 = the default; results are
  * identical, only speed changes.  The one-launch residuals (2D P1-P3 and
- * Burgers P4 without DDGIC, 3D Euler P2 and P3) have one shape and ignore it.
+ * Burgers P4 without DDGIC but Navier-Stokes P1 of more than 36000 elements,
+ * 3D Euler P2 and P3) have one shape and ignore it.
  * ice_disc_set_tile sets the shape of both the FP64 and the mixed-precision
  * residual.  ice_disc_autotune times `reps` FP64 residuals at u for each tile
  * 0-2 on the stream, keeps the fastest (*best) and writes the per-residual

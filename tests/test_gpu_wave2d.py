@@ -80,3 +80,34 @@ def test_fused_stages(flux, order):
         tol = 4 * 2.0 ** -24 if fp32 else 1e-13
         err = float((u.double() - x).abs().max() / x.abs().max())
         assert err <= tol, err
+
+
+@pytest.mark.parametrize("nel", [[157, 152], [161, 150], [190, 189], [191, 189]])
+def test_ns_p1_on_many_elements(nel):
+    """P1 Navier-Stokes on both sides of the element counts from which its
+    stages (24000) and its residual (36000) take three launches: residuals and
+    in-place residuals against the oracle, an FP64 step against the oracle's,
+    an FP32 step within two roundings of a stage's increments of it."""
+    from iceicle_amd import engine
+    from oracle.oracle import Oracle
+    m, p = _mesh(nel, abi.FLUX_NAVIER_STOKES, False), _params(abi.FLUX_NAVIER_STOKES)
+    o = Oracle(m, abi.space_desc(1), p)
+    u = cases.random_state(abi.FLUX_NAVIER_STOKES, 2, o.nelem, 4, 7).astype(np.float32).astype(np.float64)
+    ref = o.residual_parallel(u)
+    space = engine.FESpace(m, 1)
+    disc = engine.ConservationLawDDG(space, p)
+    ud = torch.from_numpy(u).cuda()
+    for precision, tol in (("fp64", 1e-12), ("mixed", 2e-5)):
+        r, w = torch.full_like(ud, float("nan")), ud.clone()
+        engine.form_residual(space, disc, ud, r, precision=precision)
+        engine.form_residual(space, disc, w, w, precision=precision)
+        err = cases.rel_inf(r.cpu().numpy(), ref)
+        print(f"{nel} {precision}: {err:.1e}", flush=True)
+        assert err <= tol and torch.equal(r, w)
+    dt = 1e-6
+    v = o.rk_solve(u, kind=0, dt=dt, ntime=1)[0]
+    for x, tol in ((ud.clone(), 1e-13), (ud.float(), 4 * 2.0 ** -24)):
+        engine.ExplicitStepper(disc, abi.stepper_desc(abi.STEP_RK3_SSP, dt=dt, ntime=1)).step(x)
+        err = cases.rel_inf(x.double().cpu().numpy(), v)
+        print(f"{nel} {x.dtype} step: {err:.1e}", flush=True)
+        assert err <= tol
