@@ -80,10 +80,17 @@ __device__ __forceinline__ void cross3(const double (&a)[3], const double (&b)[3
 // read at 64^3, 697 -> 647 us; strips of 8, 32 and 64 measured 660, 640 and
 // 657 us, 48^3 steps 1.3, 0.8 and 2% slower than 16.  Layer z is
 // workgroups z n / nz .. (z + 1) n / nz; returns -1 for a slot beyond it.
+// Layers within a strip are in order by themselves, and no slots are left empty
+// then: of thin columns' slots one in sixteen held work, on a few of the CUs
+// (1 x 1 x 5000 P2 45 us, 20 in order; the three launches 41).
 #ifndef ICE_WAVE3D_STRIP
 #define ICE_WAVE3D_STRIP 16
 #endif
 constexpr unsigned WAVE3D_STRIP = ICE_WAVE3D_STRIP;
+__host__ __device__ inline unsigned strip_layers(unsigned n, int nel2) {
+    const unsigned nz = nel2 > 1 ? nel2 : 1;
+    return (n + nz - 1) / nz > WAVE3D_STRIP ? nz : 1;
+}
 inline int strip_slots(int n, int nz) { return nz * ((n + nz - 1) / nz); }
 __device__ __forceinline__ int strip_order(unsigned slot, unsigned n, unsigned nz) {
     const unsigned per = (n + nz - 1) / nz;  // workgroups of the largest layer
@@ -109,7 +116,8 @@ __global__ __launch_bounds__(256, ICE_WAVE3D_MINW) void wave3d_kernel(DevSpace S
     constexpr bool FULL = N == 4;
     using VT = typename PH::real;
     const int lane = threadIdx.x & 63, lo = lane & 3, hi = lane >> 4, el = (lane >> 2) & 3;
-    const int wg = strip_order(xcd_contiguous(blockIdx.x, gridDim.x), ((S.nelem + 3) / 4 + 3) / 4, max(S.nel[2], 1));
+    const unsigned nwg = ((S.nelem + 3) / 4 + 3) / 4;
+    const int wg = strip_order(xcd_contiguous(blockIdx.x, gridDim.x), nwg, strip_layers(nwg, S.nel[2]));
     const int wv = wg * (blockDim.x >> 6) + (threadIdx.x >> 6);
     if (wg < 0 || wv * 4 >= S.nelem) return;
     const bool own = wv * 4 + el < S.nelem;
@@ -432,7 +440,7 @@ __global__ __launch_bounds__(256, ICE_WAVE3D_MINW) void wave3d_kernel(DevSpace S
 template <int P, class PH, class UT>
 int wave3d_launch(const DevSpace& S, const typename PH::Params& ph, const DiscDev& dd, const UT* U, double* R, UT* K,
                   const StageComb<UT>& cb, hipStream_t st) {
-    const int nw = (S.nelem + 3) / 4, nblk = strip_slots((nw + 3) / 4, std::max(S.nel[2], 1));
+    const int nw = (S.nelem + 3) / 4, nwg = (nw + 3) / 4, nblk = strip_slots(nwg, strip_layers(nwg, S.nel[2]));
     if (cb.out) {  // a stage's state has the fluxes' type
         if constexpr (std::is_same<UT, typename PH::real>::value) {
             if (S.nfb > 0) wave3d_kernel<P, PH, UT, true, true><<<nblk, 256, 0, st>>>(S, ph, dd, U, R, K, cb);

@@ -46,6 +46,25 @@ def test_residual_element_remainders(order, nel, bct):
 
 
 @pytest.mark.parametrize("order", [2, 3])
+@pytest.mark.parametrize("nel,bct", [([18, 17, 3], MIXED_BCT), ([16, 16, 4], ["PERIODIC"] * 6), ([17, 31, 2], WALLS),
+                                     ([1, 1, 333], ["PERIODIC"] * 6), ([2, 3, 150], WALLS)])
+def test_layers_and_columns(order, nel, bct):
+    """Layers of more than one strip of 16 workgroups (the last one narrower,
+    layers that do not start at a workgroup) and of exactly one, thin columns."""
+    from iceicle_amd import engine
+    from oracle.oracle import Oracle
+    m, p = _mesh(nel, bct), cases.ns_params(3, flux=abi.FLUX_EULER)
+    o = Oracle(m, abi.space_desc(order), p)
+    u = cases.random_state(abi.FLUX_EULER, 3, o.nelem, o.nbasis, 7)
+    ref = o.residual_parallel(u)
+    space = engine.FESpace(m, order)
+    disc = engine.ConservationLawDDG(space, p)
+    r = torch.full((u.size,), float("nan"), dtype=torch.float64, device="cuda")
+    engine.form_residual(space, disc, torch.from_numpy(u).cuda(), r)
+    assert cases.rel_inf(r.cpu().numpy(), ref) <= 1e-12
+
+
+@pytest.mark.parametrize("order", [2, 3])
 @pytest.mark.parametrize("bct", [["PERIODIC"] * 6, MIXED_BCT])
 def test_fused_stages(order, bct):
     from iceicle_amd import engine
