@@ -877,8 +877,9 @@ int ice_disc_autotune(ice_disc* d, const double* u, double* r, int reps, int* be
     int rc = ICE_OK;
     // FP64 residual, then the mixed one (its own tile: FP32 tiles hold half
     // the bytes, so the fastest shape can differ); the one-launch kernels have
-    // one shape, timed as tile 0 and reported for all
+    // one shape, timed as tile 0 with the repetitions of all three
     const int ntile = ice::wave_covers(s->ndim, s->p, d->prm.flux, s->mesh.nelem, d->dd) ? 1 : 3;
+    const int nrep = ntile == 1 ? 3 * reps : reps;
     for (int prec = 0; prec < 2 && rc == ICE_OK; ++prec) {
         double tbest = 1e300;
         for (int tile = 0; tile < ntile && rc == ICE_OK; ++tile) {
@@ -894,14 +895,14 @@ int ice_disc_autotune(ice_disc* d, const double* u, double* r, int reps, int* be
             bool ok = true;
             for (int k = 0; k < 2 && ok; ++k) ok = once();
             ok = ok && hipEventRecord(e0, st) == hipSuccess;
-            for (int k = 0; k < reps && ok; ++k) ok = once();
+            for (int k = 0; k < nrep && ok; ++k) ok = once();
             ok = ok && hipEventRecord(e1, st) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
                  hipEventElapsedTime(&t, e0, e1) == hipSuccess;
             if (!ok) {
                 rc = fail(ICE_ERR_HIP, "autotune timing failed");
                 break;
             }
-            const double per = (double)t / reps;
+            const double per = (double)t / nrep;
             if (ms && prec == 0)
                 for (int t = tile; t < (ntile == 1 ? 3 : tile + 1); ++t) ms[t] = per;
             if (per < tbest) {

@@ -266,7 +266,7 @@ int ice_disc_set_element_viscosity(ice_disc* disc, const double* mu);
  * milliseconds to ms[3] (either may be null); then, in 2D and 3D, times the
  * mixed-precision residual the same way and keeps its fastest tile for that
  * residual.  Where one launch forms the residual, *best is 0 and ms holds its
- * one time three times.
+ * one time, over 3 reps, three times.
  * r is overwritten.  Synchronous.  No reference counterpart. */
 int ice_disc_set_tile(ice_disc* disc, int tile);
 int ice_disc_autotune(ice_disc* disc, const double* u_dev, double* r_dev, int reps, int* best, double* ms,
