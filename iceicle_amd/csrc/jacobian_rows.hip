@@ -16,8 +16,8 @@
 //
 // Perturbing every coefficient took 2 nb m fluxes a face point against
 // 2 m + m d here, and face colour by face colour the diagonal blocks were read
-// back: 2D NS P3 64 x 64 1446 us with the residual, 203 us now (the 671 MB of
-// blocks at 3.5 TB/s; a fill of that size reaches 6.5), and a tenth of the
+// back: 2D NS P3 64 x 64 1446 us with the residual, 201 us now (the 671 MB of
+// blocks at 3.3 TB/s; a fill of that size reaches 6.5), and a tenth of the
 // differencing error.
 #include <hip/hip_runtime.h>
 

@@ -17,9 +17,13 @@
 // 160 809 elements of a study's P1 to P3 and the 67 572 of its P4: 19 / 36 / 38
 // us at P1 / P2 / P3 against 49 / 74 / 45 with matrix instructions, 53 us at
 // P4 against 115 with the trace, flux, element and inverse mass launches.  P4
-// is the faster at any size (16 x 16 step 48 for 56 us, 256 x 256 127 for 327).
+// is the faster at any size (16 x 16 step 48 for 56 us, 256 x 256 127 for 327),
+// but for steps of FP32 states below 64 x 64 with boundaries (16 x 16 59 for 53,
+// 48 x 48 57 for 55): one kernel for all sizes keeps a small instance's bits in
+// a batch.
 // Vector issue and the L1's lookups of scattered neighbour lines bound it
-// about equally (each two thirds busy at P2).
+// about equally (each two thirds busy at P2).  FP32 states keep their increments
+// (stage.h) and read them back: the same study 493 us a step to FP64's 450.
 #pragma once
 #include "residual_wave2d.h"
 

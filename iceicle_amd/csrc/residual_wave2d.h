@@ -15,8 +15,10 @@
 // Measured against the trace, flux and element launches it replaces: 2D NS
 // P3 128 x 128 FP64 39.7 -> 21.1 us, mixed 131 x 97 28.3 -> 19.2 us; Burgers
 // P2 32 x 32 residual 12.2 -> 7.5 us, RK3-SSP step 60 -> 22.5 us (14 launches
-// -> 5).  Vector issue bounds it (NS: ~1500 vector and 172 matrix
-// instructions a wave, four waves per SIMD at 128 x 128).
+// -> 5).  No one unit bounds it (NS P3 128 x 128, 1011 vector and 172
+// matrix instructions a wave): vector instructions are active in 39% of the SIMD
+// cycles and the matrix units in 25%, waves wait in 41% of theirs, and 4096 waves
+// at three a SIMD are a round and a third, 2.5 resident on average.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -96,9 +98,9 @@ struct FaceSide2 {
     }
 };
 
-// Waves per SIMD the registers must allow: 3 costs NS some scratch (96 B) and
-// measured 21.2 us against 21.2 at 2 (mixed 19.2 against 20.4); 4 spills
-// 370 B: 36 us.
+// Waves per SIMD the registers must allow: 3 costs NS some scratch (80 B a lane,
+// 12 of the 21 MB written at 128 x 128) and measured 21.2 us against 21.2 at 2
+// (mixed, 32 B: 19.2 against 20.4); 4 spills 370 B: 36 us.
 #ifndef ICE_WAVE2D_MINW
 #define ICE_WAVE2D_MINW 3
 #endif

@@ -17,7 +17,7 @@
 // Measured against the trace, flux and element launches it replaces (Euler
 // P3): 64^3 FP64 2.05 -> 0.57 ms, mixed 47 x 41 x 37 425 -> 165 us, 48^3
 // RK3-SSP step 3.74 -> 1.08 ms.  It reads 1.7 and writes 0.67 GB at 64^3
-// (0.67 and 0.67 compulsory); vector issue takes 48% and the matrix units 31%
+// (0.67 and 0.67 compulsory); vector issue takes 50% and the matrix units 32%
 // of the SIMD cycles at two waves per SIMD, what 250 registers allow.
 #pragma once
 #include <hip/hip_runtime.h>
